@@ -68,12 +68,13 @@ __device__ inline uint32_t tw_wait(const uint64_t* p, uint32_t tag, int* error, 
 {
     uint64_t w = tw_load(p);
     if (uint32_t(w >> 32) == tag) return uint32_t(w);
-    uint64_t t0 = wall_clock64();
+    const uint64_t t0 = wall_clock64();
     while (true) {
-        __builtin_amdgcn_s_sleep(1);
+        // the error flag is read together with the word: one round trip per poll
+        const int err = __hip_atomic_load(error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         w = tw_load(p);
         if (uint32_t(w >> 32) == tag) return uint32_t(w);
-        if (__hip_atomic_load(error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return 0;
+        if (err != 0) return 0;
         if (wall_clock64() - t0 > 400000000ull) {
             __hip_atomic_store(error, code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return 0;
@@ -103,10 +104,11 @@ __device__ inline void tw_gather(const uint64_t* p, const int64_t (&off)[N], con
             __hip_atomic_store(error, code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             break;
         }
-        if (__hip_atomic_load(error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) break;
-        __builtin_amdgcn_s_sleep(1);
+        // the error flag is read together with the words: one round trip per poll
+        const int err = __hip_atomic_load(error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         #pragma unroll
         for (int u = 0; u < N; ++u) w[u] = tw_load(p + off[u]);
+        if (err != 0) break;
     }
     #pragma unroll
     for (int u = 0; u < N; ++u) out[u] = uint32_t(w[u]);
@@ -158,6 +160,82 @@ __device__ inline T wave_max(T v)
 {
     for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
     return v;
+}
+
+// Wave-wide argmax without cross-lane memory operations: (value, index) with
+// the largest value, ties to the smaller index; values are -1 (no candidate,
+// index 0xFFFFFFFF) or magnitudes >= 0, never NaN.  Magnitudes order like
+// their leading 32 bits as an integer, so six DPP maxima (quads, row halves,
+// rows, then the row broadcasts, which leave the wave's maximum in lane 63)
+// find the winner's leading word; lanes that share it (rare) compare the
+// rest of the value, then the index.  Results are wave-uniform.
+template <int CTRL> __device__ __forceinline__ uint32_t dpp_max(uint32_t v)
+{
+    const uint32_t o = uint32_t(__builtin_amdgcn_update_dpp(0, int(v), CTRL, 0xf, 0xf, false));
+    return o > v ? o : v;
+}
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v)
+{
+    v = dpp_max<0xB1>(v);                              // quad_perm [1,0,3,2]
+    v = dpp_max<0x4E>(v);                              // quad_perm [2,3,0,1]
+    v = dpp_max<0x141>(v);                             // row_half_mirror
+    v = dpp_max<0x140>(v);                             // row_mirror
+    v = dpp_max<0x142>(v);                             // row_bcast 15
+    v = dpp_max<0x143>(v);                             // row_bcast 31
+    return uint32_t(__builtin_amdgcn_readlane(int(v), 63));
+}
+// The maximum of lanes 0 .. 7 (every lane of a group of eight gets its group's).
+__device__ __forceinline__ uint32_t max8_u32(uint32_t v)
+{
+    v = dpp_max<0xB1>(v);
+    v = dpp_max<0x4E>(v);
+    v = dpp_max<0x141>(v);
+    return uint32_t(__builtin_amdgcn_readfirstlane(int(v)));
+}
+__device__ __forceinline__ float lane_val(float v, int lane)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+}
+__device__ __forceinline__ double lane_val(double v, int lane)
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(u)), lane));
+    const uint32_t hi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(u >> 32)), lane));
+    return __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
+}
+// The leading word of a candidate, 0 for none.
+__device__ __forceinline__ uint32_t argmax_key(float v) { return v < 0.f ? 0u : __builtin_bit_cast(uint32_t, v) + 1u; }
+__device__ __forceinline__ uint32_t argmax_key(double v)
+{
+    return v < 0.0 ? 0u : uint32_t(__builtin_bit_cast(uint64_t, v) >> 32) + 1u;
+}
+// The lane that holds the winner (some lane if there is no candidate); key =
+// the lane's argmax_key, m = the wave's maximal key.
+template <class T>
+__device__ __forceinline__ int wave_argmax_lane(T v, uint32_t idx, uint32_t key, uint32_t m)
+{
+    uint64_t eq = __ballot(key == m);
+    if (m != 0 && (eq & (eq - 1))) {
+        if constexpr (sizeof(T) == 8) {
+            const uint32_t lo = uint32_t(__builtin_bit_cast(uint64_t, v));
+            const uint32_t ml = wave_max_u32(key == m ? lo : 0u);
+            eq = __ballot(key == m && lo == ml);
+        }
+        if (eq & (eq - 1)) {
+            const bool in = (eq >> (threadIdx.x & 63)) & 1;
+            const uint32_t mi = wave_max_u32(in ? ~idx : 0u);          // the smallest index
+            eq = __ballot(in && ~idx == mi);
+        }
+    }
+    return __builtin_ctzll(eq);
+}
+template <class T>
+__device__ __forceinline__ void wave_argmax(T& v, uint32_t& idx)
+{
+    const uint32_t key = argmax_key(v);
+    const int lane = wave_argmax_lane(v, idx, key, wave_max_u32(key));
+    v = lane_val(v, lane);
+    idx = uint32_t(__builtin_amdgcn_readlane(int(idx), lane));
 }
 
 // Map a linear block id onto tiles so that the round-robin XCD dispatch

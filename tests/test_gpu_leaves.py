@@ -1,7 +1,7 @@
 """GPU tests of the one-workgroup leaf kernels at the edges of their ranges:
 the Cholesky leaf (64 x 64, four register stages of 16 rows) and the inverted
 diagonal blocks of the look-back solves (64 rows FP64, 128 rows FP32, four
-stages)."""
+stages), and the LU panel leaf (one workgroup up to 1024 or 2048 rows)."""
 import numpy as np
 import pytest
 import torch
@@ -68,3 +68,54 @@ def test_getrs_vector_block_edges(gpu, n, trans, dtype):
     r = b - U.T @ (L.T @ x[perm]) if trans else b[perm] - L @ (U @ x)
     scale = np.abs(L).sum(1).max() * np.abs(U).sum(1).max() * np.abs(x).max()
     assert np.abs(r).max() <= 16 * max(n, 2) * float(torch.finfo(dtype).eps) * scale
+
+
+@pytest.mark.parametrize("n", [3, 33, 64, 65, 255, 256, 257, 511, 513, 1023, 1025, 2047, 2049])
+def test_panel_leaf_row_edges(gpu, n):
+    """Leaf shapes by rows: the trailing panels of one factorization run
+    through every shape below n.  Pivots equal the oracle's, factors within the
+    accumulated rounding of both (the bound of the other getrf tests)."""
+    say("panel leaf n=%d" % n)
+    A = dev_rands(300 + n, n, n)
+    info, ipiv = slate_amd.getrf(A, slate_amd.Options(block_size=128))
+    LU_o, ipiv_o, info_o = oracle.getrf(oracle.rands(300 + n, n, n), nb=128, ib=16)
+    assert info == info_o == 0
+    np.testing.assert_array_equal(ipiv, ipiv_o)
+    assert np.abs(to_host(A) - LU_o).max() <= 4 * max(n, 16) * np.finfo(np.float64).eps * np.abs(LU_o).max()
+
+
+@pytest.mark.parametrize("ib", [5, 16, 32])
+@pytest.mark.parametrize("ld", [300, 301])
+def test_panel_leaf_widths(gpu, ib, ld):
+    """Leaves narrower than the register form, aligned and unaligned rows."""
+    say("panel leaf ib=%d ld=%d" % (ib, ld))
+    n = 300
+    A = slate_amd.empty_colmajor(n, n, torch.float64, ld=ld)
+    A.copy_(dev_rands(12, n, n))
+    info, ipiv = slate_amd.getrf(A, slate_amd.Options(block_size=64, inner_blocking=ib))
+    LU_o, ipiv_o, _ = oracle.getrf(oracle.rands(12, n, n), nb=64, ib=16)
+    assert info == 0
+    np.testing.assert_array_equal(ipiv, ipiv_o)
+    assert np.abs(to_host(A) - LU_o).max() <= 4 * n * np.finfo(np.float64).eps * np.abs(LU_o).max()
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+@pytest.mark.parametrize("n", [40, 700])
+def test_panel_leaf_non_finite(gpu, value, n):
+    """A non-finite entry in column 20 leaves the columns before it, their
+    pivots and their rows' U entries as they are without it."""
+    say("panel leaf n=%d with %r" % (n, value))
+    H = oracle.rands(55, n, n)
+    A = to_dev(H)
+    slate_amd.getrf(A)
+    H2 = H.copy()
+    H2[n - 3, 20] = value
+    B = to_dev(H2)
+    _, piv = slate_amd.getrf(B)
+    LU_o, piv_o, _ = oracle.getrf(H2, nb=n, ib=32)
+    np.testing.assert_array_equal(piv[:20], piv_o[:20])
+    # columns 0 .. 19: U part and multipliers as a set (the interchanges of
+    # later columns move the rows of L, and those depend on the bad value)
+    a, b = to_host(A)[:, :20], to_host(B)[:, :20]
+    np.testing.assert_array_equal(a[:20], b[:20])
+    np.testing.assert_array_equal(np.sort(a[20:], axis=0), np.sort(b[20:], axis=0))
