@@ -246,31 +246,49 @@ void gemm_kernel(GemmArgs p)
 }
 
 //------------------------------------------------------------------------------
-// FP64 product with A K-contiguous and B N-contiguous (the LU trailing update,
-// the panel and lookahead updates): the generic kernel above moves one
-// element per load and per LDS access and recomputes clamped addresses for
-// each, which measured 47 TF (60% of the FP64 MFMA peak) with about three
-// VALU instructions per MFMA.  Here:
-//  * global loads are 16-byte vectors (8 doubles per thread per operand and
-//    slice), unguarded for interior tiles;
-//  * the K order inside a 16-deep slice is permuted so that lane l's four
-//    k-steps use k = 4 (l/16) + s: its A and B fragments for the whole slice
-//    are 4 consecutive doubles (two ds_read_b128 each) — B is stored
-//    transposed in LDS ([n][k]) for that;
-//  * LDS rows are 18 doubles (144 bytes): the 16-byte fragment reads of 8
+// Product with A K-contiguous and B N-contiguous (the LU trailing updates,
+// the panel and lookahead updates, the L11^{-1} applications, the solves'
+// off-diagonal blocks).  The generic kernel above moves one element per load
+// and per LDS access and recomputes clamped addresses for each, which measured
+// 47 TF (60% of the FP64 MFMA peak) with about three VALU instructions per
+// MFMA.  Here:
+//  * global loads are 16-byte vectors, unguarded for interior tiles; the
+//    vector types are only element-aligned (global loads need no more), so an
+//    odd leading dimension takes the same path;
+//  * the K order inside a 128-byte-deep slice (16 doubles, 32 floats) is
+//    permuted so that lane l's k-steps are consecutive (FP64: k = 4 (l/16) + s,
+//    FP32: k = 8 (l/16) + s): its A and B fragments for a slice are two
+//    ds_read_b128 each — B is stored transposed in LDS ([n][k]) for that;
+//  * LDS rows are padded by 16 bytes: the 16-byte fragment reads of 8
 //    consecutive rows fall on 8 distinct bank groups.
-template <int ROLE>
+// Tiles: 128 x 128 (SL = 1 slice per stage, two workgroups per CU) where
+// there are enough of them, else 64 x 64 or 32 x 64 with SL = 2.  A product
+// with few 128 x 128 tiles is bound by one workgroup's own chain (FP64: 4096
+// MFMA cycles per slice), not by the chip; quarter tiles shorten it four
+// times.  Every tile sums a C element's products in the same order with the
+// same MFMAs, so results do not depend on the tile.
+template <class T, int BM, int BN, int SL, int ROLE>
 __global__ __launch_bounds__(256, 2)
-void gemm_f64_kernel(GemmArgs p)
+void gemm_vec_kernel(GemmArgs p)
 {
-    constexpr int BM = 128, BN = 128, BK = 16, LDP = 18;
-    __shared__ double As[2][BM * LDP];
-    __shared__ double Bt[2][BN * LDP];
+    constexpr int VE = 16 / int(sizeof(T));         // elements per vector
+    constexpr int KS = 8 * VE;                      // elements per slice
+    constexpr int BK = SL * KS, LDP = BK + VE;
+    constexpr int FM = BM / 32, FN = BN / 32;       // 16 x 16 blocks per wave (2 x 2 waves)
+    constexpr int NVA = BK / VE;                    // vectors per staged row of A
+    constexpr int AV = BM * NVA / 256;              // A vectors per thread
+    constexpr int CPT = BN * BK / 256;              // B columns per thread
+    constexpr int BV = CPT / VE;
+    typedef T vec_t __attribute__((ext_vector_type(VE)));
+    typedef T uvec_t __attribute__((ext_vector_type(VE), aligned(sizeof(T))));
+    static_assert(BM * NVA % 256 == 0 && CPT % VE == 0 && 256 % BK == 0, "tile shape");
+    __shared__ __attribute__((aligned(16))) T As[2][BM * LDP];
+    __shared__ __attribute__((aligned(16))) T Bt[2][BN * LDP];
 
     const int64_t M = p.M, N = p.N, K = p.K;
     const int64_t tiles_m = ceildiv(M, BM), tiles_n = ceildiv(N, BN);
     // uplo with a square tile grid: only the upper-triangle tiles are launched
-    const bool tri = p.uplo == 1 && tiles_m == tiles_n;
+    const bool tri = p.uplo == 1 && BM == BN && tiles_m == tiles_n;
     const int64_t ntiles = tri ? tiles_m * (tiles_m + 1) / 2 : tiles_m * tiles_n;
     int64_t t = xcd_remap(blockIdx.x, ntiles);
     int64_t m0, n0;
@@ -291,59 +309,70 @@ void gemm_f64_kernel(GemmArgs p)
     }
     if (p.uplo == 1 && n0 + BN <= m0) return;
 
-    const double* __restrict__ A = static_cast<const double*>(p.A);
-    const double* __restrict__ B = static_cast<const double*>(p.B);
-    double* __restrict__ C = static_cast<double*>(p.C);
+    const T* __restrict__ A = static_cast<const T*>(p.A);
+    const T* __restrict__ B = static_cast<const T*>(p.B);
+    T* __restrict__ C = static_cast<T*>(p.C);
     const int64_t lda = p.lda, ldb = p.ldb, ldc = p.ldc;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int fr = lane & 15, fk = lane >> 4;
-    // staging: A row ar, k ak .. ak+7; B k row bk, columns bc .. bc+7
-    const int ar = tid >> 1, ak = (tid & 1) * 8;
-    const int bk = tid & 15, bc = (tid >> 4) * 8;
+    // staging: A vector u of this thread is vector (tid + 256 u) % NVA of row
+    // (tid + 256 u) / NVA; B k row bk, columns bc .. bc + CPT - 1
+    const int bk = tid % BK, bc = (tid / BK) * CPT;
     const bool full_mn = m0 + BM <= M && n0 + BN <= N;
-    const bool vec_ok = (lda % 2 == 0) && (ldb % 2 == 0) && (reinterpret_cast<uintptr_t>(A) % 16 == 0)
-                        && (reinterpret_cast<uintptr_t>(B) % 16 == 0);
-    double ra[8], rb[8];
+    vec_t ra[AV], rb[BV];
     auto load = [&](int64_t k0) {
-        if (full_mn && vec_ok && k0 + BK <= K) {
-            const double* ap = A + (m0 + ar) * lda + k0 + ak;
-            const double* bp = B + (k0 + bk) * ldb + n0 + bc;
+        if (full_mn && k0 + BK <= K) {
+            const T* bp = B + (k0 + bk) * ldb + n0 + bc;
             #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const v2d x = *reinterpret_cast<const v2d*>(ap + 2 * q);
-                const v2d y = *reinterpret_cast<const v2d*>(bp + 2 * q);
-                ra[2 * q] = x[0]; ra[2 * q + 1] = x[1];
-                rb[2 * q] = y[0]; rb[2 * q + 1] = y[1];
+            for (int u = 0; u < AV; ++u) {
+                const int e = tid + 256 * u;
+                ra[u] = *reinterpret_cast<const uvec_t*>(A + (m0 + e / NVA) * lda + k0 + (e % NVA) * VE);
             }
+            #pragma unroll
+            for (int u = 0; u < BV; ++u) rb[u] = *reinterpret_cast<const uvec_t*>(bp + u * VE);
         }
         else {
-            const int64_t gmr = m0 + ar, gkb = k0 + bk;
-            const int64_t cm = gmr < M ? gmr : M - 1, ckb = gkb < K ? gkb : K - 1;
             #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int64_t gk = k0 + ak + e, gn = n0 + bc + e;
-                const double x = A[cm * lda + (gk < K ? gk : K - 1)];
-                const double y = B[ckb * ldb + (gn < N ? gn : N - 1)];
-                ra[e] = (gmr < M && gk < K) ? x : 0.0;
-                rb[e] = (gkb < K && gn < N) ? y : 0.0;
+            for (int u = 0; u < AV; ++u) {
+                const int e = tid + 256 * u;
+                const int64_t gmr = m0 + e / NVA, cm = gmr < M ? gmr : M - 1;
+                #pragma unroll
+                for (int f = 0; f < VE; ++f) {
+                    const int64_t gk = k0 + (e % NVA) * VE + f;
+                    const T x = A[cm * lda + (gk < K ? gk : K - 1)];
+                    ra[u][f] = (gmr < M && gk < K) ? x : T(0);
+                }
             }
+            const int64_t gkb = k0 + bk, ckb = gkb < K ? gkb : K - 1;
+            #pragma unroll
+            for (int u = 0; u < BV; ++u)
+                #pragma unroll
+                for (int f = 0; f < VE; ++f) {
+                    const int64_t gn = n0 + bc + u * VE + f;
+                    const T y = B[ckb * ldb + (gn < N ? gn : N - 1)];
+                    rb[u][f] = (gkb < K && gn < N) ? y : T(0);
+                }
         }
     };
     auto store = [&](int buf) {
         #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            *reinterpret_cast<v2d*>(&As[buf][ar * LDP + ak + 2 * q]) = v2d{ra[2 * q], ra[2 * q + 1]};
+        for (int u = 0; u < AV; ++u) {
+            const int e = tid + 256 * u;
+            *reinterpret_cast<vec_t*>(&As[buf][(e / NVA) * LDP + (e % NVA) * VE]) = ra[u];
+        }
         #pragma unroll
-        for (int e = 0; e < 8; ++e) Bt[buf][(bc + e) * LDP + bk] = rb[e];
+        for (int c = 0; c < CPT; ++c) Bt[buf][(bc + c) * LDP + bk] = rb[c / VE][c % VE];
     };
 
-    v4d acc[4][4];
+    typename Mf<T>::acc acc[FM][FN];
     #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < FM; ++i)
         #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+        for (int j = 0; j < FN; ++j)
+            #pragma unroll
+            for (int r = 0; r < 4; ++r) acc[i][j][r] = T(0);
 
     const int64_t ktiles = ceildiv(K, BK);
     load(0);
@@ -353,23 +382,23 @@ void gemm_f64_kernel(GemmArgs p)
         const int cur = int(kt & 1);
         const bool more = kt + 1 < ktiles;
         if (more) load((kt + 1) * BK);
-        // two k-step pairs: each lane's fragments for a pair are one 16-byte read
+        // half slices: each lane's fragments for one are one 16-byte read
         #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            v2d af[4], bf[4];
+        for (int h = 0; h < 2 * SL; ++h) {
+            const int ko = (h / 2) * KS + (KS / 4) * fk + VE * (h % 2);
+            vec_t af[FM], bf[FN];
             #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                af[i] = *reinterpret_cast<const v2d*>(&As[cur][(wm * 64 + i * 16 + fr) * LDP + 4 * fk + 2 * h]);
+            for (int i = 0; i < FM; ++i)
+                af[i] = *reinterpret_cast<const vec_t*>(&As[cur][(wm * (BM / 2) + i * 16 + fr) * LDP + ko]);
             #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                bf[j] = *reinterpret_cast<const v2d*>(&Bt[cur][(wn * 64 + j * 16 + fr) * LDP + 4 * fk + 2 * h]);
+            for (int j = 0; j < FN; ++j)
+                bf[j] = *reinterpret_cast<const vec_t*>(&Bt[cur][(wn * (BN / 2) + j * 16 + fr) * LDP + ko]);
             #pragma unroll
-            for (int s_ = 0; s_ < 2; ++s_)
+            for (int s_ = 0; s_ < VE; ++s_)
                 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+                for (int i = 0; i < FM; ++i)
                     #pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i][s_], bf[j][s_], acc[i][j], 0, 0, 0);
+                    for (int j = 0; j < FN; ++j) acc[i][j] = Mf<T>::op(af[i][s_], bf[j][s_], acc[i][j]);
         }
         if (more) {
             store(cur ^ 1);
@@ -377,211 +406,58 @@ void gemm_f64_kernel(GemmArgs p)
         }
     }
 
-    const double alpha = p.alpha, beta = p.beta;
-    // Interior tiles: each 16-row block reads its 16 C values per lane with
-    // no per-element branches, so they are in flight together (the guarded
+    const T alpha = T(p.alpha), beta = T(p.beta);
+    // Interior tiles: each 16-row block reads its C values with no
+    // per-element branches, so they are in flight together (the guarded
     // element-by-element form below waits one memory round trip per element).
-    const bool full = m0 + BM <= M && n0 + BN <= N && (p.uplo == 0 || n0 >= m0 + BM);
+    const bool full = full_mn && (p.uplo == 0 || n0 >= m0 + BM);
     if (full) {
-        double* cb = C + (m0 + wm * 64 + fk) * ldc + n0 + wn * 64 + fr;
+        T* cb = C + (m0 + wm * (BM / 2)) * ldc + n0 + wn * (BN / 2) + fr;
         #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            double cv[4][4];
+        for (int i = 0; i < FM; ++i) {
+            T cv[FN][4];
             #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < FN; ++j)
                 #pragma unroll
-                for (int r = 0; r < 4; ++r) cv[j][r] = beta != 0.0 ? cb[(i * 16 + 4 * r) * ldc + j * 16] : 0.0;
+                for (int r = 0; r < 4; ++r)
+                    cv[j][r] = beta != T(0) ? cb[(i * 16 + Mf<T>::row(lane, r)) * ldc + j * 16] : T(0);
             #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < FN; ++j)
                 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    double v = alpha * acc[i][j][r];
-                    if (beta != 0.0) v += beta * cv[j][r];
-                    cb[(i * 16 + 4 * r) * ldc + j * 16] = v;
+                    T v = alpha * acc[i][j][r];
+                    if (beta != T(0)) v += beta * cv[j][r];
+                    cb[(i * 16 + Mf<T>::row(lane, r)) * ldc + j * 16] = v;
                 }
         }
         return;
     }
     #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < FM; ++i)
         #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < FN; ++j)
             #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int64_t gm_ = m0 + wm * 64 + i * 16 + 4 * r + fk;
-                const int64_t gn_ = n0 + wn * 64 + j * 16 + fr;
+                const int64_t gm_ = m0 + wm * (BM / 2) + i * 16 + Mf<T>::row(lane, r);
+                const int64_t gn_ = n0 + wn * (BN / 2) + j * 16 + fr;
                 if (gm_ < M && gn_ < N && (p.uplo == 0 || gn_ >= gm_)) {
-                    double* c = C + gm_ * ldc + gn_;
-                    double v = alpha * acc[i][j][r];
-                    if (beta != 0.0) v += beta * *c;
+                    T* c = C + gm_ * ldc + gn_;
+                    T v = alpha * acc[i][j][r];
+                    if (beta != T(0)) v += beta * *c;
                     *c = v;
                 }
             }
 }
 
-//------------------------------------------------------------------------------
-// FP32 product with A K-contiguous and B N-contiguous (the float LU's
-// L11^{-1} applications, the panel's node updates, the solves' off-diagonal
-// blocks, and the trailing update of the FP32-MFMA factor): the FP64 kernel
-// above with float operands and v_mfma_f32_16x16x4f32.  Slices are 32 deep
-// (the same 128-byte rows), lane l's eight k-steps use k = 8 (l/16) + s, so
-// its A and B fragments for a slice are 8 consecutive floats (two
-// ds_read_b128 each); LDS rows are 36 floats (144 bytes) as in the FP64
-// kernel.  The accumulator layout differs from FP64's: register r of lane l
-// holds D[4 (l/16) + r][l%16].
-template <int ROLE>
-__global__ __launch_bounds__(256, 2)
-void gemm_f32_kernel(GemmArgs p)
+template <class T, int BM, int BN, int SL, int ROLE>
+static void launch_vec(const GemmArgs& a, hipStream_t s)
 {
-    constexpr int BM = 128, BN = 128, BK = 32, LDP = 36;
-    __shared__ float As[2][BM * LDP];
-    __shared__ float Bt[2][BN * LDP];
-
-    const int64_t M = p.M, N = p.N, K = p.K;
-    const int64_t tiles_m = ceildiv(M, BM), tiles_n = ceildiv(N, BN);
-    // uplo with a square tile grid: only the upper-triangle tiles are launched
-    const bool tri = p.uplo == 1 && tiles_m == tiles_n;
-    const int64_t ntiles = tri ? tiles_m * (tiles_m + 1) / 2 : tiles_m * tiles_n;
-    int64_t t = xcd_remap(blockIdx.x, ntiles);
-    int64_t m0, n0;
-    if (tri) {
-        int64_t tm, tn;
-        upper_tile(t, tiles_m, tm, tn);
-        m0 = tm * BM;
-        n0 = tn * BN;
-    }
-    else {
-        constexpr int64_t GM = 8;
-        int64_t group = t / (GM * tiles_n);
-        int64_t first_m = group * GM;
-        int64_t gm = (tiles_m - first_m < GM) ? (tiles_m - first_m) : GM;
-        int64_t within = t - group * GM * tiles_n;
-        m0 = (first_m + within % gm) * BM;
-        n0 = (within / gm) * BN;
-    }
-    if (p.uplo == 1 && n0 + BN <= m0) return;
-
-    const float* __restrict__ A = static_cast<const float*>(p.A);
-    const float* __restrict__ B = static_cast<const float*>(p.B);
-    float* __restrict__ C = static_cast<float*>(p.C);
-    const int64_t lda = p.lda, ldb = p.ldb, ldc = p.ldc;
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int fr = lane & 15, fk = lane >> 4;
-    // staging: A row ar, k ak .. ak+15; B k row bk, columns bc .. bc+15
-    const int ar = tid >> 1, ak = (tid & 1) * 16;
-    const int bk = tid & 31, bc = (tid >> 5) * 16;
-    const bool full_mn = m0 + BM <= M && n0 + BN <= N;
-    const bool vec_ok = (lda % 4 == 0) && (ldb % 4 == 0) && (reinterpret_cast<uintptr_t>(A) % 16 == 0)
-                        && (reinterpret_cast<uintptr_t>(B) % 16 == 0);
-    v4f ra[4], rb[4];
-    auto load = [&](int64_t k0) {
-        if (full_mn && vec_ok && k0 + BK <= K) {
-            const float* ap = A + (m0 + ar) * lda + k0 + ak;
-            const float* bp = B + (k0 + bk) * ldb + n0 + bc;
-            #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                ra[q] = *reinterpret_cast<const v4f*>(ap + 4 * q);
-                rb[q] = *reinterpret_cast<const v4f*>(bp + 4 * q);
-            }
-        }
-        else {
-            const int64_t gmr = m0 + ar, gkb = k0 + bk;
-            const int64_t cm = gmr < M ? gmr : M - 1, ckb = gkb < K ? gkb : K - 1;
-            #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int64_t gk = k0 + ak + e, gn = n0 + bc + e;
-                const float x = A[cm * lda + (gk < K ? gk : K - 1)];
-                const float y = B[ckb * ldb + (gn < N ? gn : N - 1)];
-                ra[e >> 2][e & 3] = (gmr < M && gk < K) ? x : 0.0f;
-                rb[e >> 2][e & 3] = (gkb < K && gn < N) ? y : 0.0f;
-            }
-        }
-    };
-    auto store = [&](int buf) {
-        #pragma unroll
-        for (int q = 0; q < 4; ++q) *reinterpret_cast<v4f*>(&As[buf][ar * LDP + ak + 4 * q]) = ra[q];
-        #pragma unroll
-        for (int e = 0; e < 16; ++e) Bt[buf][(bc + e) * LDP + bk] = rb[e >> 2][e & 3];
-    };
-
-    v4f acc[4][4];
-    #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-
-    const int64_t ktiles = ceildiv(K, BK);
-    load(0);
-    store(0);
-    __syncthreads();
-    for (int64_t kt = 0; kt < ktiles; ++kt) {
-        const int cur = int(kt & 1);
-        const bool more = kt + 1 < ktiles;
-        if (more) load((kt + 1) * BK);
-        #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            v4f af[4], bf[4];
-            #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                af[i] = *reinterpret_cast<const v4f*>(&As[cur][(wm * 64 + i * 16 + fr) * LDP + 8 * fk + 4 * h]);
-            #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                bf[j] = *reinterpret_cast<const v4f*>(&Bt[cur][(wn * 64 + j * 16 + fr) * LDP + 8 * fk + 4 * h]);
-            #pragma unroll
-            for (int s_ = 0; s_ < 4; ++s_)
-                #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    #pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i][s_], bf[j][s_], acc[i][j], 0, 0, 0);
-        }
-        if (more) {
-            store(cur ^ 1);
-            __syncthreads();
-        }
-    }
-
-    const float alpha = float(p.alpha), beta = float(p.beta);
-    // Interior tiles: C read per 16-row block with no per-element branches
-    // (see gemm_f64_kernel).
-    const bool full = m0 + BM <= M && n0 + BN <= N && (p.uplo == 0 || n0 >= m0 + BM);
-    if (full) {
-        float* cb = C + (m0 + wm * 64 + 4 * fk) * ldc + n0 + wn * 64 + fr;
-        #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float cv[4][4];
-            #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                #pragma unroll
-                for (int r = 0; r < 4; ++r) cv[j][r] = beta != 0.0f ? cb[(i * 16 + r) * ldc + j * 16] : 0.0f;
-            #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    float v = alpha * acc[i][j][r];
-                    if (beta != 0.0f) v += beta * cv[j][r];
-                    cb[(i * 16 + r) * ldc + j * 16] = v;
-                }
-        }
-        return;
-    }
-    #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int64_t gm_ = m0 + wm * 64 + i * 16 + 4 * fk + r;
-                const int64_t gn_ = n0 + wn * 64 + j * 16 + fr;
-                if (gm_ < M && gn_ < N && (p.uplo == 0 || gn_ >= gm_)) {
-                    float* c = C + gm_ * ldc + gn_;
-                    float v = alpha * acc[i][j][r];
-                    if (beta != 0.0f) v += beta * *c;
-                    *c = v;
-                }
-            }
+    const int64_t tm = ceildiv(a.M, BM), tn = ceildiv(a.N, BN);
+    // only the upper-triangle tiles of a square triangular update
+    const int64_t nt = a.uplo == 1 && BM == BN && tm == tn ? tm * (tm + 1) / 2 : tm * tn;
+    SA_REQUIRE(nt < (int64_t(1) << 31), -2, "gemm: grid too large");
+    hipLaunchKernelGGL((gemm_vec_kernel<T, BM, BN, SL, ROLE>), dim3(unsigned(nt)), dim3(256), 0, s, a);
+    SA_CHECK_LAUNCH();
 }
 
 //------------------------------------------------------------------------------
@@ -685,27 +561,29 @@ static void launch(const GemmArgs& a, hipStream_t s)
             return;
         }
     }
-    // 128 x 128 tiles, 4 waves, two workgroups per CU (2 waves per SIMD) —
-    // the fastest of the tilings measured for both FP64 and FP32.
-    constexpr int BM = 128, BN = 128, BK = (sizeof(T) == 8) ? 16 : 32;
-    int64_t nt = ceildiv(a.M, BM) * ceildiv(a.N, BN);
-    // the 16-byte-staged kernels launch only the upper-triangle tiles of a
-    // square triangular update (same tile size in both directions)
-    if constexpr (ALAY == A_KC && BLAY == B_NC)
-        if (a.uplo == 1 && ceildiv(a.M, BM) == ceildiv(a.N, BN))
-            nt = ceildiv(a.M, BM) * (ceildiv(a.M, BM) + 1) / 2;
-    SA_REQUIRE(nt < (int64_t(1) << 31), -2, "gemm: grid too large");
-    if constexpr (std::is_same<T, double>::value && ALAY == A_KC && BLAY == B_NC) {
-        hipLaunchKernelGGL((gemm_f64_kernel<ROLE>), dim3(unsigned(nt)), dim3(256), 0, s, a);
-    }
-    else if constexpr (std::is_same<T, float>::value && ALAY == A_KC && BLAY == B_NC) {
-        hipLaunchKernelGGL((gemm_f32_kernel<ROLE>), dim3(unsigned(nt)), dim3(256), 0, s, a);
+    if constexpr (ALAY == A_KC && BLAY == B_NC) {
+        // From one 128 x 128 tile per CU on the large tile is as fast as any
+        // (FP64 2048^2 x 256 55 us, 64 x 64 53 us; 31000^2 x 768 61 and 54
+        // TF).  Below that the chip is idle and the chain of one tile sets
+        // the time: FP64 1900 x 128 x 128 44 us with 128 x 128, 17 us with
+        // 64 x 64, 12 us with 32 x 64; 8000 x 256 x 256 85, 28 and 35 us;
+        // FP32 8000 x 256 x 256 61, 18 and 22 us.  32 x 64 wins while the
+        // 64 x 64 tiles do not fill the CUs either (4096 x 64 x 4096: 1190,
+        // 177 and 119 us).
+        const int64_t nt128 = ceildiv(a.M, 128) * ceildiv(a.N, 128), nt64 = ceildiv(a.M, 64) * ceildiv(a.N, 64);
+        if (nt128 >= 256) launch_vec<T, 128, 128, 1, ROLE>(a, s);
+        else if (a.uplo == 1 || nt64 >= 256) launch_vec<T, 64, 64, 2, ROLE>(a, s);
+        else launch_vec<T, 32, 64, 2, ROLE>(a, s);
     }
     else {
+        // 128 x 128 tiles, 4 waves, two workgroups per CU
+        constexpr int BM = 128, BN = 128, BK = (sizeof(T) == 8) ? 16 : 32;
+        const int64_t nt = ceildiv(a.M, BM) * ceildiv(a.N, BN);
+        SA_REQUIRE(nt < (int64_t(1) << 31), -2, "gemm: grid too large");
         hipLaunchKernelGGL((gemm_kernel<T, ALAY, BLAY, BM, BN, BK, 2, 2, 2, ROLE>), dim3(unsigned(nt)), dim3(256),
                            0, s, a);
+        SA_CHECK_LAUNCH();
     }
-    SA_CHECK_LAUNCH();
 }
 
 template <class T>

@@ -119,3 +119,26 @@ def test_panel_leaf_non_finite(gpu, value, n):
     a, b = to_host(A)[:, :20], to_host(B)[:, :20]
     np.testing.assert_array_equal(a[:20], b[:20])
     np.testing.assert_array_equal(np.sort(a[20:], axis=0), np.sort(b[20:], axis=0))
+
+
+# 32 x 64 tiles (few tiles), 64 x 64 and 128 x 128 tiles, each with whole
+# tiles, ragged edges, a k tail, and operands one element off 16-byte alignment
+@pytest.mark.parametrize("m,n,k", [(70, 130, 200), (64, 128, 128), (1100, 1000, 70), (1088, 1024, 64),
+                                   (2100, 2050, 33), (2048, 2176, 48)])
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_gemm_tiles(gpu, m, n, k, off, dtype):
+    """|computed - exact| <= (k + 2) eps (|A| |B| + |C|), entry by entry."""
+    say("gemm tiles %dx%dx%d off=%d %s" % (m, n, k, off, dtype))
+    g = torch.Generator("cuda").manual_seed(m + n + k)
+
+    def mat(r, c):
+        S = torch.empty(c, r + 3, dtype=dtype, device="cuda").uniform_(-1, 1, generator=g).t()
+        return S[off:off + r]
+
+    A, B, C = mat(m, k), mat(k, n), mat(m, n)
+    a, b, c0 = A.double(), B.double(), C.double().clone()
+    slate_amd.gemm(-1.0, A, B, 0.5, C)
+    ref = 0.5 * c0 - a @ b
+    bound = (k + 2) * float(torch.finfo(dtype).eps) * (a.abs() @ b.abs() + 0.5 * c0.abs())
+    assert bool(((C.double() - ref).abs() <= bound).all())
