@@ -96,7 +96,7 @@ struct Context {
     unsigned char* scratch = nullptr;   // this device's no-allocation scratch (noalloc.hip)
     Buf swaptmp;                 // two-pass row interchange workspace (trailing-update stream)
     Buf swaptmp1;                // the same for the lookahead block (tall blocks only)
-    Buf ttri;                    // row-major copy of a column-major-view triangle (Cholesky solves)
+    Buf ttri;                    // diagonal block of a solve with few right-hand sides, row-major
     Buf cut0, cut1;              // Cholesky: K-contiguous U12^T for the trailing (s0) and block-row (s1) updates
     uint32_t tv_tag = 0;         // next free tag of tvw
     bool calu = false;           // leaves use tournament pivoting (MethodLU::CALU)
@@ -262,18 +262,27 @@ static void check_kernel_error(Context& c)
 // Recursive triangular solve with an nb x nb triangle and an nb x N row-major
 // right-hand side; off-diagonal blocks go through the MFMA GEMM.
 // tri(i,k) = M[i*ld + k] (cm = 0) or M[i + k*ld] (cm = 1).
+// tri (TRSM_TRI^2 elements, or null) is for solves with few right-hand sides
+// against a large triangle: diagonal blocks of at most TRSM_TRI rows, which a
+// column-major view copies there row-major.  With 64 right-hand sides a
+// 512-row block in one launch has 8 workgroups and takes 245 us read by
+// columns; two of 256 rows and the product between them take about 80.
+constexpr int64_t TRSM_TRI = 256;
 template <class T>
 static void trsm_rec(const T* M, int64_t ld, int cm, int lower, int unit, int64_t nb,
-                     T* B, int64_t ldb, int64_t N, hipStream_t s)
+                     T* B, int64_t ldb, int64_t N, hipStream_t s, T* tri = nullptr)
 {
     if (nb <= 0 || N <= 0) return;
     constexpr int64_t L = TRSM_LEAF;
     if (nb <= L) { trsm_leaf<T>(M, ld, cm, lower, unit, nb, B, ldb, N, s); return; }
-    // the lower row-major solves (the panel's, L11^{-1}, getrs' L sweep, the
-    // Cholesky blocks after their transposed copy) run as one launch up to
-    // trsm_fused_max rows
-    if (cm == 0 && lower && nb <= trsm_fused_max(int(sizeof(T)))) {
-        trsm_lower_fused<T>(M, ld, nb, B, ldb, N, unit, s);
+    if (nb <= (tri ? TRSM_TRI : trsm_fused_max(int(sizeof(T))))) {
+        if (tri && cm) {
+            transpose_convert<T, T>(M, ld, tri, nb, nb, nb, s);        // tri[i*nb + k] = M[i + k*ld]
+            trsm_fused<T>(tri, nb, 0, lower, unit, nb, B, ldb, N, s);
+        }
+        else {
+            trsm_fused<T>(M, ld, cm, lower, unit, nb, B, ldb, N, s);
+        }
         return;
     }
     int64_t n1 = ((nb / 2 + L - 1) / L) * L;
@@ -286,39 +295,23 @@ static void trsm_rec(const T* M, int64_t ld, int cm, int lower, int unit, int64_
     GemmArgs g{};
     g.alpha = -1.0; g.beta = 1.0; g.uplo = 0;
     if (lower) {
-        trsm_rec<T>(M11, ld, cm, 1, unit, n1, B1, ldb, N, s);
+        trsm_rec<T>(M11, ld, cm, 1, unit, n1, B1, ldb, N, s, tri);
         // B2 -= tri(n1:, 0:n1) * B1
         g.M = n2; g.N = N; g.K = n1;
         g.A = cm ? static_cast<const void*>(M + n1) : static_cast<const void*>(M + n1 * ld);
         g.lda = ld; g.B = B1; g.ldb = ldb; g.C = B2; g.ldc = ldb;
         gemm<T>(g, cm ? A_MC : A_KC, B_NC, s);
-        trsm_rec<T>(M22, ld, cm, 1, unit, n2, B2, ldb, N, s);
+        trsm_rec<T>(M22, ld, cm, 1, unit, n2, B2, ldb, N, s, tri);
     }
     else {
-        trsm_rec<T>(M22, ld, cm, 0, unit, n2, B2, ldb, N, s);
+        trsm_rec<T>(M22, ld, cm, 0, unit, n2, B2, ldb, N, s, tri);
         // B1 -= tri(0:n1, n1:) * B2
         g.M = n1; g.N = N; g.K = n2;
         g.A = cm ? static_cast<const void*>(M + n1 * ld) : static_cast<const void*>(M + n1);
         g.lda = ld; g.B = B2; g.ldb = ldb; g.C = B1; g.ldc = ldb;
         gemm<T>(g, cm ? A_MC : A_KC, B_NC, s);
-        trsm_rec<T>(M11, ld, cm, 0, unit, n1, B1, ldb, N, s);
+        trsm_rec<T>(M11, ld, cm, 0, unit, n1, B1, ldb, N, s, tri);
     }
-}
-
-// Lower triangle of a column-major view (cm = 1: tri(i, k) = M[i + k*ld], the
-// transposed row-major upper factor of the Cholesky): copied row-major into
-// c.ttri (nb^2 elements) so that the one-launch lower solve applies; false
-// when the triangle is outside that solve's range.
-template <class T>
-static bool trsm_lower_cm_fused(Context& c, const T* M, int64_t ld, int unit, int64_t nb, T* B, int64_t ldb,
-                                int64_t N, hipStream_t s)
-{
-    if (nb <= TRSM_LEAF || nb > trsm_fused_max(int(sizeof(T))) || N <= 0) return false;
-    c.ttri.ensure(sizeof(T) * size_t(nb) * size_t(nb));
-    T* Lr = c.ttri.as<T>();
-    transpose_convert<T, T>(M, ld, Lr, nb, nb, nb, s);               // Lr[i*nb + k] = M[i + k*ld]
-    trsm_lower_fused<T>(Lr, nb, nb, B, ldb, N, unit, s);
-    return true;
 }
 
 // Wide triangular solve B := tri^{-1} B for an nb x nb triangle and an
@@ -333,8 +326,7 @@ static void trsm_wide(Context& c, const T* M, int64_t ld, int cm, int lower, int
                       T* B, int64_t ldb, int64_t N, hipStream_t s)
 {
     if (N < 4 * nb || nb <= TRSM_LEAF) {
-        if (!(cm == 1 && lower && trsm_lower_cm_fused<T>(c, M, ld, unit, nb, B, ldb, N, s)))
-            trsm_rec<T>(M, ld, cm, lower, unit, nb, B, ldb, N, s);
+        trsm_rec<T>(M, ld, cm, lower, unit, nb, B, ldb, N, s);
         return;
     }
     c.tinv.ensure(sizeof(T) * size_t(nb) * size_t(nb));
@@ -342,8 +334,7 @@ static void trsm_wide(Context& c, const T* M, int64_t ld, int cm, int lower, int
     T* inv = c.tinv.as<T>();
     T* tmp = c.ttmp.as<T>();
     set_identity<T>(inv, nb, nb, s);
-    if (!(cm == 1 && lower && trsm_lower_cm_fused<T>(c, M, ld, unit, nb, inv, nb, nb, s)))
-        trsm_rec<T>(M, ld, cm, lower, unit, nb, inv, nb, nb, s);
+    trsm_rec<T>(M, ld, cm, lower, unit, nb, inv, nb, nb, s);
     GemmArgs g{};
     g.M = nb; g.N = N; g.K = nb;
     g.A = inv; g.lda = nb; g.B = B; g.ldb = ldb; g.C = tmp; g.ldc = N;
@@ -410,13 +401,13 @@ static void unit_lower_inverse(const T* L, int64_t ld, int64_t nb, T* inv, hipSt
         trsm_rec<T>(L, ld, 0, 1, 1, nb, inv, nb, nb, s);
         return;
     }
-    trsm_lunit_fused<T>(L, ld, h, inv, nb, h, s);                       // X11
+    trsm_fused<T>(L, ld, 0, 1, 1, h, inv, nb, h, s);                    // X11
     GemmArgs g{};
     g.M = h2; g.N = h; g.K = h;
     g.A = L + h * ld; g.lda = ld; g.B = inv; g.ldb = nb; g.C = inv + h * nb; g.ldc = nb;
     g.alpha = -1.0; g.beta = 0.0; g.uplo = 0;
     gemm<T>(g, A_KC, B_NC, s);                                          // -L21 X11
-    trsm_lunit_fused<T>(L + h * ld + h, ld, h2, inv + h * nb, nb, nb, s);  // [X21 X22]
+    trsm_fused<T>(L + h * ld + h, ld, 0, 1, 1, h2, inv + h * nb, nb, nb, s);  // [X21 X22]
 }
 
 //------------------------------------------------------------------------------
@@ -822,8 +813,7 @@ static void potrf_diag_rec(Context& c, T* M, int64_t ld, int64_t nb, int64_t col
     if (n1 >= nb) n1 = nb - 64;
     int64_t n2 = nb - n1;
     potrf_diag_rec<T>(c, M, ld, n1, col0, info, s);
-    if (!trsm_lower_cm_fused<T>(c, M, ld, 0, n1, M + n1, ld, n2, s))
-        trsm_rec<T>(M, ld, 1, 1, 0, n1, M + n1, ld, n2, s);
+    trsm_rec<T>(M, ld, 1, 1, 0, n1, M + n1, ld, n2, s);
     GemmArgs g{};
     g.M = n2; g.N = n2; g.K = n1;
     g.A = M + n1; g.lda = ld; g.B = M + n1; g.ldb = ld;
@@ -861,7 +851,7 @@ static void potrf_rm(Context& c, T* A, int64_t n, int64_t ld, const Opts& o, int
     // Lookahead as in the LU (src/potrf.cc:84-194 with Option::Lookahead): s1
     // applies step k to the next block row and factors it (diagonal block and
     // row-panel solve), while s0 applies step k to the rows beyond it.  The
-    // panel's workspaces (tinv, ttmp, ttri) belong to s1; s0 uses cut0.
+    // panel's workspaces (tinv, ttmp) belong to s1; s0 uses cut0.
     const bool la = o.lookahead > 0 && nsteps > 2;
     hipStream_t s0 = c.s0, s1 = la ? c.s1 : c.s0;
     if (int64_t(c.evs.size()) < 2 * nsteps + 4) {
@@ -1043,28 +1033,34 @@ static T* dinv_pair(Context& c, int64_t n)
     return c.dinv.as<T>();
 }
 
-// Single right-hand side: x := op(LU)^{-1} x with x contiguous, using the
-// one-launch look-back triangular solves.  perm is the getrf permutation.
+// Most right-hand sides solved one by one with the look-back sweeps: each
+// costs a read of the factors, the blocked solve a fixed chain of launches.
+constexpr int64_t VEC_RHS_MAX = 4;
+
+// Few right-hand sides: X := op(LU)^{-1} X column by column (ldx apart, each
+// contiguous), using the one-launch look-back triangular solves; tmp holds n.
+// perm is the getrf permutation.
 template <class T>
 static void getrs_vec(Context& c, const T* LU, int64_t ld, int cm, int64_t n, const int64_t* perm,
-                      T* x, T* tmp, int trans, hipStream_t s)
+                      T* X, int64_t ldx, int64_t nrhs, T* tmp, int trans, hipStream_t s)
 {
     T* d0 = dinv_pair<T>(c, n);
     T* d1 = d0 + trsv_aux_elems(n, int(sizeof(T)));
-    if (!trans) {
-        trsv_diag_inverse<T>(LU, ld, cm, 1, 1, n, d0, s);
-        trsv_diag_inverse<T>(LU, ld, cm, 0, 0, n, d1, s);
-        permute_convert<T, T>(x, tmp, perm, n, 0, s);
-        trsv_lookback<T>(LU, ld, cm, 1, n, d0, tmp, tv_next(c, n), s);
-        trsv_lookback<T>(LU, ld, cm, 0, n, d1, tmp, tv_next(c, n), s);
-        copy_convert<T, T>(tmp, n, x, n, n, 1, s);
-    }
-    else {
-        trsv_diag_inverse<T>(LU, ld, 1 - cm, 1, 0, n, d0, s);
-        trsv_diag_inverse<T>(LU, ld, 1 - cm, 0, 1, n, d1, s);
-        trsv_lookback<T>(LU, ld, 1 - cm, 1, n, d0, x, tv_next(c, n), s);
-        trsv_lookback<T>(LU, ld, 1 - cm, 0, n, d1, x, tv_next(c, n), s);
-        permute_convert<T, T>(x, tmp, perm, n, 1, s);
+    const int t = trans ? 1 - cm : cm;                  // A^T = U^T L^T P^T: U^T is the lower one
+    trsv_diag_inverse<T>(LU, ld, t, 1, trans ? 0 : 1, n, d0, s);
+    trsv_diag_inverse<T>(LU, ld, t, 0, trans ? 1 : 0, n, d1, s);
+    for (int64_t j = 0; j < nrhs; ++j) {
+        T* x = X + j * ldx;
+        if (!trans) {
+            permute_convert<T, T>(x, tmp, perm, n, 0, s);
+            trsv_lookback<T>(LU, ld, t, 1, n, d0, tmp, tv_next(c, n), s);
+            trsv_lookback<T>(LU, ld, t, 0, n, d1, tmp, tv_next(c, n), s);
+        }
+        else {
+            trsv_lookback<T>(LU, ld, t, 1, n, d0, x, tv_next(c, n), s);
+            trsv_lookback<T>(LU, ld, t, 0, n, d1, x, tv_next(c, n), s);
+            permute_convert<T, T>(x, tmp, perm, n, 1, s);
+        }
         copy_convert<T, T>(tmp, n, x, n, n, 1, s);
     }
 }
@@ -1074,17 +1070,19 @@ static void getrs_any(Context& c, const T* LU, int64_t ld, int cm, int64_t n, co
                       T* B, int64_t ldb, int64_t nrhs, int trans, hipStream_t s)
 {
     c.plan0.ensure(sizeof(int64_t) * (4 * 2048 + 8));
+    c.ttri.ensure(sizeof(T) * size_t(TRSM_TRI * TRSM_TRI));
     int64_t* plan = c.plan0.as<int64_t>();
+    T* tri = c.ttri.as<T>();
     if (!trans) {
         for (int64_t k1 = 0; k1 < n; k1 += 1024)
             laswp<T>(B, ldb, n, 0, nrhs, k1, std::min(n, k1 + 1024), ipiv, plan, s);
-        trsm_rec<T>(LU, ld, cm, 1, 1, n, B, ldb, nrhs, s);
-        trsm_rec<T>(LU, ld, cm, 0, 0, n, B, ldb, nrhs, s);
+        trsm_rec<T>(LU, ld, cm, 1, 1, n, B, ldb, nrhs, s, tri);
+        trsm_rec<T>(LU, ld, cm, 0, 0, n, B, ldb, nrhs, s, tri);
     }
     else {
         // A^T = U^T L^T P^T: solve U^T then L^T (transposed access), then P.
-        trsm_rec<T>(LU, ld, 1 - cm, 1, 0, n, B, ldb, nrhs, s);
-        trsm_rec<T>(LU, ld, 1 - cm, 0, 1, n, B, ldb, nrhs, s);
+        trsm_rec<T>(LU, ld, 1 - cm, 1, 0, n, B, ldb, nrhs, s, tri);
+        trsm_rec<T>(LU, ld, 1 - cm, 0, 1, n, B, ldb, nrhs, s, tri);
         // interchanges applied backward (src/getrs.cc:106-114): chunks from the
         // end, each as the inverse of its forward (dst <- src) plan
         for (int64_t k2 = n; k2 > 0; k2 -= 1024) {
@@ -1096,12 +1094,15 @@ static void getrs_any(Context& c, const T* LU, int64_t ld, int cm, int64_t n, co
     }
 }
 
-// Solve with the row-major upper Cholesky factor: U^T y = b, U x = y.
+// Solve with a Cholesky factor as a row-major upper triangle U (cm = 0:
+// U^T y = b, U x = y) or a row-major lower one (cm = 1, U its transpose).
 template <class T>
-static void potrs_rm(const T* U, int64_t ld, int64_t n, T* B, int64_t ldb, int64_t nrhs, hipStream_t s)
+static void potrs_rm(Context& c, const T* U, int64_t ld, int cm, int64_t n, T* B, int64_t ldb, int64_t nrhs,
+                     hipStream_t s)
 {
-    trsm_rec<T>(U, ld, 1, 1, 0, n, B, ldb, nrhs, s);
-    trsm_rec<T>(U, ld, 0, 0, 0, n, B, ldb, nrhs, s);
+    c.ttri.ensure(sizeof(T) * size_t(TRSM_TRI * TRSM_TRI));
+    trsm_rec<T>(U, ld, 1 - cm, 1, 0, n, B, ldb, nrhs, s, c.ttri.as<T>());
+    trsm_rec<T>(U, ld, cm, 0, 0, n, B, ldb, nrhs, s, c.ttri.as<T>());
 }
 
 //------------------------------------------------------------------------------
@@ -1241,13 +1242,13 @@ template <class T>
 static void getrs_cm(Context& c, int trans, const T* A, int64_t lda, int64_t n, const int64_t* d_ipiv,
                      T* B, int64_t ldb, int64_t nrhs)
 {
-    if (nrhs == 1) {
+    if (nrhs <= VEC_RHS_MAX) {
         std::vector<int64_t> ip(n);
         SA_HIP(hipMemcpyAsync(ip.data(), d_ipiv, sizeof(int64_t) * n, hipMemcpyDeviceToHost, c.s0));
         SA_HIP(hipStreamSynchronize(c.s0));
         const int64_t* perm = upload_perm(c, ip.data(), n);
         c.rhs.ensure(sizeof(T) * size_t(n));
-        getrs_vec<T>(c, A, lda, 1, n, perm, B, c.rhs.as<T>(), trans, c.s0);
+        getrs_vec<T>(c, A, lda, 1, n, perm, B, ldb, nrhs, c.rhs.as<T>(), trans, c.s0);
         SA_HIP(hipStreamSynchronize(c.s0));
         check_kernel_error(c);
         return;
@@ -1273,7 +1274,7 @@ static int64_t potrf_cm(Context& c, int uplo, T* A, int64_t n, int64_t lda, cons
 template <class T>
 static void potrs_cm(Context& c, int uplo, T* A, int64_t lda, int64_t n, T* B, int64_t ldb, int64_t nrhs)
 {
-    if (nrhs == 1) {
+    if (nrhs <= VEC_RHS_MAX) {
         // Lower column-major L (A = L L^T): L y = b, L^T x = y.
         // Upper column-major U (A = U^T U): U^T y = b, U x = y.
         const int cmL = (uplo == SLATE_AMD_UPPER) ? 0 : 1;
@@ -1281,21 +1282,17 @@ static void potrs_cm(Context& c, int uplo, T* A, int64_t lda, int64_t n, T* B, i
         T* d1 = d0 + trsv_aux_elems(n, int(sizeof(T)));
         trsv_diag_inverse<T>(A, lda, cmL, 1, 0, n, d0, c.s0);
         trsv_diag_inverse<T>(A, lda, 1 - cmL, 0, 0, n, d1, c.s0);
-        trsv_lookback<T>(A, lda, cmL, 1, n, d0, B, tv_next(c, n), c.s0);
-        trsv_lookback<T>(A, lda, 1 - cmL, 0, n, d1, B, tv_next(c, n), c.s0);
+        for (int64_t j = 0; j < nrhs; ++j) {
+            trsv_lookback<T>(A, lda, cmL, 1, n, d0, B + j * ldb, tv_next(c, n), c.s0);
+            trsv_lookback<T>(A, lda, 1 - cmL, 0, n, d1, B + j * ldb, tv_next(c, n), c.s0);
+        }
         SA_HIP(hipStreamSynchronize(c.s0));
         check_kernel_error(c);
         return;
     }
     T* W = rhs_rm<T>(c, c.rhs, B, ldb, n, nrhs);
-    if (uplo == SLATE_AMD_UPPER) {
-        // column-major upper U (A = U^T U) is row-major lower U^T
-        trsm_rec<T>(A, lda, 0, 1, 0, n, W, nrhs, nrhs, c.s0);
-        trsm_rec<T>(A, lda, 1, 0, 0, n, W, nrhs, nrhs, c.s0);
-    }
-    else {
-        potrs_rm<T>(A, lda, n, W, nrhs, nrhs, c.s0);
-    }
+    // column-major upper U (A = U^T U) is row-major lower U^T
+    potrs_rm<T>(c, A, lda, uplo == SLATE_AMD_UPPER ? 1 : 0, n, W, nrhs, nrhs, c.s0);
     rhs_back<T>(c, W, B, ldb, n, nrhs);
 }
 
@@ -1360,7 +1357,7 @@ static double norm_host(Context& c, const double* A, int64_t n, int64_t lda, int
 
 static void lo_solve(Context& c, const MixedState& st, int sym, int64_t n, int64_t nrhs)
 {
-    if (sym) potrs_rm<float>(st.Alo, n, n, st.xlo, nrhs, nrhs, c.s0);
+    if (sym) potrs_rm<float>(c, st.Alo, n, 0, n, st.xlo, nrhs, nrhs, c.s0);
     else getrs_any<float>(c, st.Alo, n, 0, n, st.ipiv, st.xlo, nrhs, nrhs, 0, c.s0);
 }
 

@@ -246,9 +246,9 @@ void gemm_kernel(GemmArgs p)
 }
 
 //------------------------------------------------------------------------------
-// Product with A K-contiguous and B N-contiguous (the LU trailing updates,
-// the panel and lookahead updates, the L11^{-1} applications, the solves'
-// off-diagonal blocks).  The generic kernel above moves one element per load
+// Product with B N-contiguous, A either way (the LU trailing updates, the
+// panel and lookahead updates, the L11^{-1} applications; with A M-contiguous
+// the solves and Cholesky blocks on a column-major view).  The generic kernel above moves one element per load
 // and per LDS access and recomputes clamped addresses for each, which measured
 // 47 TF (60% of the FP64 MFMA peak) with about three VALU instructions per
 // MFMA.  Here:
@@ -267,7 +267,7 @@ void gemm_kernel(GemmArgs p)
 // MFMA cycles per slice), not by the chip; quarter tiles shorten it four
 // times.  Every tile sums a C element's products in the same order with the
 // same MFMAs, so results do not depend on the tile.
-template <class T, int BM, int BN, int SL, int ROLE>
+template <class T, int ALAY, int BM, int BN, int SL, int ROLE>
 __global__ __launch_bounds__(256, 2)
 void gemm_vec_kernel(GemmArgs p)
 {
@@ -279,6 +279,7 @@ void gemm_vec_kernel(GemmArgs p)
     constexpr int AV = BM * NVA / 256;              // A vectors per thread
     constexpr int CPT = BN * BK / 256;              // B columns per thread
     constexpr int BV = CPT / VE;
+    constexpr int RPT = BM * BK / 256;              // A rows per thread (A_MC)
     typedef T vec_t __attribute__((ext_vector_type(VE)));
     typedef T uvec_t __attribute__((ext_vector_type(VE), aligned(sizeof(T))));
     static_assert(BM * NVA % 256 == 0 && CPT % VE == 0 && 256 % BK == 0, "tile shape");
@@ -317,9 +318,10 @@ void gemm_vec_kernel(GemmArgs p)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int fr = lane & 15, fk = lane >> 4;
-    // staging: A vector u of this thread is vector (tid + 256 u) % NVA of row
-    // (tid + 256 u) / NVA; B k row bk, columns bc .. bc + CPT - 1
-    const int bk = tid % BK, bc = (tid / BK) * CPT;
+    // staging: A_KC vector u of this thread is vector (tid + 256 u) % NVA of
+    // row (tid + 256 u) / NVA; B k row bk, columns bc .. bc + CPT - 1, and
+    // A_MC likewise column bk, rows ar .. ar + RPT - 1 (both transposed into LDS)
+    const int bk = tid % BK, bc = (tid / BK) * CPT, ar = (tid / BK) * RPT;
     const bool full_mn = m0 + BM <= M && n0 + BN <= N;
     vec_t ra[AV], rb[BV];
     auto load = [&](int64_t k0) {
@@ -328,7 +330,9 @@ void gemm_vec_kernel(GemmArgs p)
             #pragma unroll
             for (int u = 0; u < AV; ++u) {
                 const int e = tid + 256 * u;
-                ra[u] = *reinterpret_cast<const uvec_t*>(A + (m0 + e / NVA) * lda + k0 + (e % NVA) * VE);
+                const T* ap = ALAY == A_KC ? A + (m0 + e / NVA) * lda + k0 + (e % NVA) * VE
+                                           : A + (k0 + bk) * lda + m0 + ar + u * VE;
+                ra[u] = *reinterpret_cast<const uvec_t*>(ap);
             }
             #pragma unroll
             for (int u = 0; u < BV; ++u) rb[u] = *reinterpret_cast<const uvec_t*>(bp + u * VE);
@@ -337,12 +341,13 @@ void gemm_vec_kernel(GemmArgs p)
             #pragma unroll
             for (int u = 0; u < AV; ++u) {
                 const int e = tid + 256 * u;
-                const int64_t gmr = m0 + e / NVA, cm = gmr < M ? gmr : M - 1;
                 #pragma unroll
                 for (int f = 0; f < VE; ++f) {
-                    const int64_t gk = k0 + (e % NVA) * VE + f;
-                    const T x = A[cm * lda + (gk < K ? gk : K - 1)];
-                    ra[u][f] = (gmr < M && gk < K) ? x : T(0);
+                    const int64_t gm_ = ALAY == A_KC ? m0 + e / NVA : m0 + ar + u * VE + f;
+                    const int64_t gk = ALAY == A_KC ? k0 + (e % NVA) * VE + f : k0 + bk;
+                    const int64_t cm = gm_ < M ? gm_ : M - 1, ck = gk < K ? gk : K - 1;
+                    const T x = A[ALAY == A_KC ? cm * lda + ck : ck * lda + cm];
+                    ra[u][f] = (gm_ < M && gk < K) ? x : T(0);
                 }
             }
             const int64_t gkb = k0 + bk, ckb = gkb < K ? gkb : K - 1;
@@ -357,10 +362,16 @@ void gemm_vec_kernel(GemmArgs p)
         }
     };
     auto store = [&](int buf) {
-        #pragma unroll
-        for (int u = 0; u < AV; ++u) {
-            const int e = tid + 256 * u;
-            *reinterpret_cast<vec_t*>(&As[buf][(e / NVA) * LDP + (e % NVA) * VE]) = ra[u];
+        if constexpr (ALAY == A_KC) {
+            #pragma unroll
+            for (int u = 0; u < AV; ++u) {
+                const int e = tid + 256 * u;
+                *reinterpret_cast<vec_t*>(&As[buf][(e / NVA) * LDP + (e % NVA) * VE]) = ra[u];
+            }
+        }
+        else {
+            #pragma unroll
+            for (int c = 0; c < RPT; ++c) As[buf][(ar + c) * LDP + bk] = ra[c / VE][c % VE];
         }
         #pragma unroll
         for (int c = 0; c < CPT; ++c) Bt[buf][(bc + c) * LDP + bk] = rb[c / VE][c % VE];
@@ -449,14 +460,14 @@ void gemm_vec_kernel(GemmArgs p)
             }
 }
 
-template <class T, int BM, int BN, int SL, int ROLE>
+template <class T, int ALAY, int BM, int BN, int SL, int ROLE>
 static void launch_vec(const GemmArgs& a, hipStream_t s)
 {
     const int64_t tm = ceildiv(a.M, BM), tn = ceildiv(a.N, BN);
     // only the upper-triangle tiles of a square triangular update
     const int64_t nt = a.uplo == 1 && BM == BN && tm == tn ? tm * (tm + 1) / 2 : tm * tn;
     SA_REQUIRE(nt < (int64_t(1) << 31), -2, "gemm: grid too large");
-    hipLaunchKernelGGL((gemm_vec_kernel<T, BM, BN, SL, ROLE>), dim3(unsigned(nt)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((gemm_vec_kernel<T, ALAY, BM, BN, SL, ROLE>), dim3(unsigned(nt)), dim3(256), 0, s, a);
     SA_CHECK_LAUNCH();
 }
 
@@ -561,7 +572,7 @@ static void launch(const GemmArgs& a, hipStream_t s)
             return;
         }
     }
-    if constexpr (ALAY == A_KC && BLAY == B_NC) {
+    if constexpr (BLAY == B_NC) {
         // From one 128 x 128 tile per CU on the large tile is as fast as any
         // (FP64 2048^2 x 256 55 us, 64 x 64 53 us; 31000^2 x 768 61 and 54
         // TF).  Below that the chip is idle and the chain of one tile sets
@@ -571,12 +582,12 @@ static void launch(const GemmArgs& a, hipStream_t s)
         // 64 x 64 tiles do not fill the CUs either (4096 x 64 x 4096: 1190,
         // 177 and 119 us).
         const int64_t nt128 = ceildiv(a.M, 128) * ceildiv(a.N, 128), nt64 = ceildiv(a.M, 64) * ceildiv(a.N, 64);
-        if (nt128 >= 256) launch_vec<T, 128, 128, 1, ROLE>(a, s);
-        else if (a.uplo == 1 || nt64 >= 256) launch_vec<T, 64, 64, 2, ROLE>(a, s);
-        else launch_vec<T, 32, 64, 2, ROLE>(a, s);
+        if (nt128 >= 256) launch_vec<T, ALAY, 128, 128, 1, ROLE>(a, s);
+        else if (a.uplo == 1 || nt64 >= 256) launch_vec<T, ALAY, 64, 64, 2, ROLE>(a, s);
+        else launch_vec<T, ALAY, 32, 64, 2, ROLE>(a, s);
     }
     else {
-        // 128 x 128 tiles, 4 waves, two workgroups per CU
+        // B K-contiguous: the test matrix generator's products only
         constexpr int BM = 128, BN = 128, BK = (sizeof(T) == 8) ? 16 : 32;
         const int64_t nt = ceildiv(a.M, BM) * ceildiv(a.N, BN);
         SA_REQUIRE(nt < (int64_t(1) << 31), -2, "gemm: grid too large");

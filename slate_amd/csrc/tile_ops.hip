@@ -109,22 +109,29 @@ template void trsm_leaf<float>(const float*, int64_t, int, int, int, int64_t, fl
                                int64_t, hipStream_t);
 
 //------------------------------------------------------------------------------
-// L X = B in place for a lower triangle (tri(i, k) = L[i*ldl + k], m x m;
-// unit diagonal or not) and a row-major B (m x N, ldb), in one launch,
-// m <= trsm_fused_max.
+// tri X = B in place for an m x m triangle (lower or upper, unit diagonal or
+// not, row- or column-major view) and a row-major B (m x N, ldb), in one
+// launch, m <= trsm_fused_max.  An upper triangle is the lower one of the
+// reversed index: the kernel sees tri(i, k) = L[i*rs + k*cs] and rows of B
+// bs apart, with negative strides for it.
 // Workgroup x owns the columns [8x, 8x + 8), kept in LDS k-contiguous.  The
 // sweep is left-looking over 32-row blocks: every thread owns one (row,
 // column) of the block and forms y = b - L(i, 0:p0) X(0:p0, c) from LDS; then
 // the block's forward substitution runs in registers, each wave holding two
 // columns (one per 32-lane half) and broadcasting each solved entry with
 // v_readlane.  The block row L(p0:p0+32, 0:p0+32) reaches LDS in chunks of
-// 32 rows x 512 bytes, each loaded once per workgroup with coalesced 16-byte
-// loads (consecutive threads read consecutive pieces of a row) and the next
-// chunk's loads in flight while the current one is multiplied.  Reading the
-// row straight from memory instead, one row per lane, makes every load touch
-// 32 rows and leaves the kernel bound by address processing (1.7-2x slower,
-// the same sums).  Two barriers per chunk, no launches inside the sweep: the
-// recursive form needs 2 m/32 - 1 launches.
+// 32 rows x 512 bytes, each loaded once per workgroup with coalesced loads
+// (16 bytes along a row, or 32 rows of a column) and the next chunk's loads
+// in flight while the current one is multiplied.  Reading the row straight
+// from memory instead, one row per lane, makes every load touch 32 rows and
+// leaves the kernel bound by address processing (1.7-2x slower, the same
+// sums).  Two barriers per chunk, no launches inside the sweep: the recursive
+// form needs 2 m/32 - 1 launches.
+// Non-unit diagonals: 32 dependent divisions per block are as long as the
+// rest of the substitution, so each row's reciprocal is formed once, off the
+// chain, and the quotient is corrected by its residual, which rounds as the
+// division does; blocks with a diagonal entry outside the range where that
+// holds divide.
 template <class T> __device__ __forceinline__ T bcast_half(T v, int k, bool upper);
 template <> __device__ __forceinline__ float bcast_half<float>(float v, int k, bool upper)
 {
@@ -151,18 +158,21 @@ template <> struct Vec16<double> { typedef double __attribute__((ext_vector_type
 
 template <class T>
 struct TrsmProb {
-    const T* L; int64_t ldl; T* B; int64_t ldb; int64_t N; int m; int ldx; int vec_ok;
+    const T* L; int64_t rs, cs; T* B; int64_t bs; int64_t N; int m; int ldx;
 };
 
 // 16-byte vectors per row of a staged chunk of the block row
 static constexpr int TRSM_NV = 32;
 
-template <class T, int UNIT>
+// CONT: 1 row entries contiguous (cs = 1), -1 the same reversed (cs = -1),
+// 0 column entries contiguous (rs = 1 or -1)
+template <class T, int UNIT, int CONT>
 __global__ __launch_bounds__(256)
-void trsm_lunit_kernel(TrsmProb<T> P)
+void trsm_fused_kernel(TrsmProb<T> P)
 {
     typedef typename Vec16<T>::type V;
     constexpr int VN = Vec16<T>::n;
+    typedef T UV __attribute__((ext_vector_type(VN), aligned(sizeof(T))));
     constexpr int NV = TRSM_NV;
     constexpr int KC = NV * VN;                         // columns per chunk
     constexpr int LP = KC + VN;                         // padded chunk row pitch
@@ -171,7 +181,7 @@ void trsm_lunit_kernel(TrsmProb<T> P)
     if (j0 >= P.N) return;                              // uniform per workgroup, before any barrier
     const T* __restrict__ L = P.L;
     T* __restrict__ B = P.B;
-    const int64_t ldl = P.ldl, ldb = P.ldb, N = P.N;
+    const int64_t rs = P.rs, cs = P.cs, bs = P.bs, N = P.N;
     const int m = P.m, ldx = P.ldx;
     extern __shared__ __align__(16) unsigned char trsm_lds[];
     T* Xs = reinterpret_cast<T*>(trsm_lds);            // column c at Xs + c*ldx
@@ -184,26 +194,44 @@ void trsm_lunit_kernel(TrsmProb<T> P)
         const int c = tid & 7;
         const bool cv = j0 + c < N;
         for (int i = tid >> 3; i < m; i += 32)
-            Xs[c * ldx + i] = cv ? B[int64_t(i) * ldb + j0 + c] : T(0);
+            Xs[c * ldx + i] = cv ? B[int64_t(i) * bs + j0 + c] : T(0);
     }
     T* Xc = Xs + cl * ldx;
     const V* Lr = reinterpret_cast<const V*>(Lc + r * LP);
-    // chunk (q0, kc): rows [q0, q0 + 32), columns [kc, kc + KC), strictly-lower
-    // entries only (zeros elsewhere), into registers
+    // chunk (q0, kc): rows [q0, q0 + 32), columns [kc, kc + KC), lower entries
+    // only (zeros elsewhere), into registers; loads are clamped, not guarded
     V pv[NU];
     auto fetch = [&](int q0, int kc) {
         #pragma unroll
         for (int u = 0; u < NU; ++u) {
-            const int e = tid + 256 * u;
-            const int col = kc + (e % NV) * VN, row = q0 + e / NV;
-            #pragma unroll
-            for (int t = 0; t < VN; ++t) pv[u][t] = T(0);
-            if (row < m && col < row) {
-                const T* src = L + int64_t(row) * ldl + col;
-                if (P.vec_ok && col + VN <= row) pv[u] = *reinterpret_cast<const V*>(src);
+            if constexpr (CONT != 0) {
+                const int e = tid + 256 * u;
+                const int col = kc + (e % NV) * VN, row = q0 + e / NV;
+                const int cr = row < m ? row : m - 1;
+                if (kc + KC <= m) {
+                    const T* src = L + int64_t(cr) * rs + int64_t(col) * cs;
+                    if constexpr (CONT > 0) pv[u] = *reinterpret_cast<const UV*>(src);
+                    else {
+                        const V x = *reinterpret_cast<const UV*>(src - (VN - 1));
+                        #pragma unroll
+                        for (int t = 0; t < VN; ++t) pv[u][t] = x[VN - 1 - t];
+                    }
+                }
                 else {
                     #pragma unroll
-                    for (int t = 0; t < VN; ++t) if (col + t < row) pv[u][t] = src[t];
+                    for (int t = 0; t < VN; ++t)
+                        pv[u][t] = L[int64_t(cr) * rs + int64_t(col + t < m ? col + t : m - 1) * cs];
+                }
+                #pragma unroll
+                for (int t = 0; t < VN; ++t) pv[u][t] = (row < m && col + t <= row) ? pv[u][t] : T(0);
+            }
+            else {
+                #pragma unroll
+                for (int t = 0; t < VN; ++t) {
+                    const int e = tid + 256 * (u * VN + t);
+                    const int row = q0 + (e & 31), col = kc + (e >> 5);
+                    const T x = L[int64_t(row < m ? row : m - 1) * rs + int64_t(col < m ? col : m - 1) * cs];
+                    pv[u][t] = (row < m && col <= row) ? x : T(0);
                 }
             }
         }
@@ -214,14 +242,23 @@ void trsm_lunit_kernel(TrsmProb<T> P)
         T acc[VN];
         #pragma unroll
         for (int e = 0; e < VN; ++e) acc[e] = T(0);
-        T lr[32];
+        T lr[32], diag = T(1);
         // chunks cover columns [0, p0 + 32); the last one holds the diagonal block
         for (int kc = 0; kc < p0 + 32; kc += KC) {
             __syncthreads();                            // previous chunk consumed, X rows written
             #pragma unroll
             for (int u = 0; u < NU; ++u) {
-                const int e = tid + 256 * u;
-                *reinterpret_cast<V*>(Lc + (e / NV) * LP + (e % NV) * VN) = pv[u];
+                if constexpr (CONT != 0) {
+                    const int e = tid + 256 * u;
+                    *reinterpret_cast<V*>(Lc + (e / NV) * LP + (e % NV) * VN) = pv[u];
+                }
+                else {
+                    #pragma unroll
+                    for (int t = 0; t < VN; ++t) {
+                        const int e = tid + 256 * (u * VN + t);
+                        Lc[(e & 31) * LP + (e >> 5)] = pv[u][t];
+                    }
+                }
             }
             __syncthreads();
             {
@@ -241,6 +278,7 @@ void trsm_lunit_kernel(TrsmProb<T> P)
                 const T* d = Lc + r * LP + (p0 - kc);
                 #pragma unroll
                 for (int k = 0; k < 32; ++k) lr[k] = d[k];
+                if (!UNIT && i < m) diag = d[r];
             }
         }
         T y = T(0);
@@ -250,61 +288,83 @@ void trsm_lunit_kernel(TrsmProb<T> P)
             for (int e = 1; e < VN; ++e) sum += acc[e];
             y = Xc[i] - sum;
         }
-        const T diag = (!UNIT && i < m) ? L[int64_t(i) * ldl + i] : T(1);
-        #pragma unroll
-        for (int k = 0; k < 31; ++k) {
-            if (!UNIT && r == k) y = y / diag;
-            const T xk = bcast_half<T>(y, k, upper);
-            if (r > k) y -= lr[k] * xk;
+        if constexpr (UNIT) {
+            #pragma unroll
+            for (int k = 0; k < 31; ++k) {
+                const T xk = bcast_half<T>(y, k, upper);
+                if (r > k) y -= lr[k] * xk;
+            }
         }
-        if (!UNIT && r == 31) y = y / diag;
+        else {
+            constexpr T big = sizeof(T) == 8 ? T(1e290) : T(1e30);
+            const T inv = T(1) / diag;
+            if (__ballot(!(fabs(diag) < big && fabs(inv) < big)) == 0) {
+                #pragma unroll
+                for (int k = 0; k < 32; ++k) {
+                    const T q0 = y * inv;
+                    const T q1 = fma(fma(-q0, diag, y), inv, q0);
+                    if (r == k) y = isfinite(q1) ? q1 : q0;
+                    if (k < 31) {
+                        const T xk = bcast_half<T>(y, k, upper);
+                        if (r > k) y -= lr[k] * xk;
+                    }
+                }
+            }
+            else {
+                #pragma unroll
+                for (int k = 0; k < 32; ++k) {
+                    if (r == k) y = y / diag;
+                    if (k < 31) {
+                        const T xk = bcast_half<T>(y, k, upper);
+                        if (r > k) y -= lr[k] * xk;
+                    }
+                }
+            }
+        }
         if (i < m) Xc[i] = y;
     }
     __syncthreads();
     {
         const int c = tid & 7;
         if (j0 + c < N)
-            for (int i = tid >> 3; i < m; i += 32) B[int64_t(i) * ldb + j0 + c] = Xs[c * ldx + i];
+            for (int i = tid >> 3; i < m; i += 32) B[int64_t(i) * bs + j0 + c] = Xs[c * ldx + i];
     }
 }
 
 int64_t trsm_fused_max(int elem_bytes) { return elem_bytes == 8 ? 768 : 1024; }
 
 template <class T>
-static TrsmProb<T> trsm_prob(const T* L, int64_t ldl, int64_t m, T* B, int64_t ldb, int64_t N, size_t& lds)
-{
-    SA_REQUIRE(m <= trsm_fused_max(int(sizeof(T))), -2, "trsm_lunit_fused: triangle too large");
-    SA_REQUIRE(ceildiv(N, 8) < (int64_t(1) << 31), -2, "trsm_lunit_fused: too many columns");
-    constexpr int VN = Vec16<T>::n;
-    TrsmProb<T> q;
-    q.L = L; q.ldl = ldl; q.B = B; q.ldb = ldb; q.N = N; q.m = int(m);
-    q.ldx = int(ceildiv(m, 32) * 32) + VN;
-    q.vec_ok = (reinterpret_cast<uintptr_t>(L) % 16 == 0 && ldl % VN == 0) ? 1 : 0;
-    lds = std::max(lds, sizeof(T) * (size_t(8) * size_t(q.ldx) + 32 * size_t(TRSM_NV * VN + VN)));
-    return q;
-}
-
-template <class T>
-void trsm_lower_fused(const T* L, int64_t ldl, int64_t m, T* B, int64_t ldb, int64_t N, int unit, hipStream_t s)
+void trsm_fused(const T* M, int64_t ld, int cm, int lower, int unit, int64_t m, T* B, int64_t ldb, int64_t N,
+                hipStream_t s)
 {
     if (m <= 0 || N <= 0) return;
-    size_t lds = 0;
-    const TrsmProb<T> q = trsm_prob(L, ldl, m, B, ldb, N, lds);
-    if (unit) hipLaunchKernelGGL((trsm_lunit_kernel<T, 1>), dim3(unsigned(ceildiv(N, 8))), dim3(256), lds, s, q);
-    else hipLaunchKernelGGL((trsm_lunit_kernel<T, 0>), dim3(unsigned(ceildiv(N, 8))), dim3(256), lds, s, q);
+    SA_REQUIRE(m <= trsm_fused_max(int(sizeof(T))), -2, "trsm_fused: triangle too large");
+    SA_REQUIRE(ceildiv(N, 8) < (int64_t(1) << 31), -2, "trsm_fused: too many columns");
+    constexpr int VN = Vec16<T>::n;
+    TrsmProb<T> q;
+    q.rs = cm ? 1 : ld;
+    q.cs = cm ? ld : 1;
+    q.bs = ldb;
+    q.L = M;
+    q.B = B;
+    if (!lower) {                                       // the reversed index
+        q.L = M + (m - 1) * (ld + 1);
+        q.B = B + (m - 1) * ldb;
+        q.rs = -q.rs; q.cs = -q.cs; q.bs = -q.bs;
+    }
+    q.N = N; q.m = int(m);
+    q.ldx = int(ceildiv(m, 32) * 32) + VN;
+    const size_t lds = sizeof(T) * (size_t(8) * size_t(q.ldx) + 32 * size_t(TRSM_NV * VN + VN));
+    const dim3 grid(unsigned(ceildiv(N, 8))), blk(256);
+#define SA_TRSM_FUSED(U, C) hipLaunchKernelGGL((trsm_fused_kernel<T, U, C>), grid, blk, lds, s, q)
+    if (unit) { if (cm) SA_TRSM_FUSED(1, 0); else if (lower) SA_TRSM_FUSED(1, 1); else SA_TRSM_FUSED(1, -1); }
+    else { if (cm) SA_TRSM_FUSED(0, 0); else if (lower) SA_TRSM_FUSED(0, 1); else SA_TRSM_FUSED(0, -1); }
+#undef SA_TRSM_FUSED
     SA_CHECK_LAUNCH();
 }
 
-template <class T>
-void trsm_lunit_fused(const T* L, int64_t ldl, int64_t m, T* B, int64_t ldb, int64_t N, hipStream_t s)
-{
-    trsm_lower_fused<T>(L, ldl, m, B, ldb, N, 1, s);
-}
-
-template void trsm_lower_fused<double>(const double*, int64_t, int64_t, double*, int64_t, int64_t, int, hipStream_t);
-template void trsm_lower_fused<float>(const float*, int64_t, int64_t, float*, int64_t, int64_t, int, hipStream_t);
-template void trsm_lunit_fused<double>(const double*, int64_t, int64_t, double*, int64_t, int64_t, hipStream_t);
-template void trsm_lunit_fused<float>(const float*, int64_t, int64_t, float*, int64_t, int64_t, hipStream_t);
+template void trsm_fused<double>(const double*, int64_t, int, int, int, int64_t, double*, int64_t, int64_t, hipStream_t);
+template void trsm_fused<float>(const float*, int64_t, int, int, int, int64_t, float*, int64_t, int64_t, hipStream_t);
 //------------------------------------------------------------------------------
 // Right-looking upper Cholesky (A = U^T U) of one nb x nb block, nb <= 64.
 // Row-major upper == column-major lower, so this is LAPACK's lower dpotrf on

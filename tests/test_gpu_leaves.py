@@ -142,3 +142,61 @@ def test_gemm_tiles(gpu, m, n, k, off, dtype):
     ref = 0.5 * c0 - a @ b
     bound = (k + 2) * float(torch.finfo(dtype).eps) * (a.abs() @ b.abs() + 0.5 * c0.abs())
     assert bool(((C.double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("n", [33, 64, 257, 300, 700])
+@pytest.mark.parametrize("nrhs", [2, 5, 9])
+@pytest.mark.parametrize("trans", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_getrs_matrix_edges(gpu, n, nrhs, trans, dtype):
+    """Several right-hand sides: column by column up to four, blocked beyond;
+    both triangles in both views.  Same factors and bound as the vector test."""
+    say("getrs n=%d nrhs=%d trans=%s %s" % (n, nrhs, trans, dtype))
+    F = 0.5 * oracle.rands(90 + n, n, n) / n
+    F[np.arange(n), np.arange(n)] = 1.5 + 0.5 * oracle.rands(91, n, 1)[:, 0]
+    A = to_dev(F, dtype)
+    F = to_host(A)
+    L = np.tril(F, -1) + np.eye(n)
+    U = np.triu(F)
+    ipiv = np.arange(1, n + 1)
+    ipiv[0] = n
+    B = dev_rands(92, n, nrhs, dtype)
+    b = to_host(B)
+    slate_amd.getrs(A, ipiv, B, trans=trans)
+    x = to_host(B)
+    perm = np.arange(n)
+    perm[0], perm[n - 1] = perm[n - 1], perm[0]
+    r = b - U.T @ (L.T @ x[perm]) if trans else b[perm] - L @ (U @ x)
+    scale = np.abs(L).sum(1).max() * np.abs(U).sum(1).max() * np.abs(x).max()
+    assert np.abs(r).max() <= 16 * n * float(torch.finfo(dtype).eps) * scale
+
+
+@pytest.mark.parametrize("n", [40, 300, 1000])
+@pytest.mark.parametrize("nrhs", [4, 6])
+@pytest.mark.parametrize("uplo", [slate_amd.LOWER, slate_amd.UPPER])
+def test_posv_matrix_edges(gpu, n, nrhs, uplo):
+    say("posv n=%d nrhs=%d uplo=%d" % (n, nrhs, uplo))
+    S = spd(4, n)
+    A = to_dev(S)
+    B = dev_rands(5, n, nrhs)
+    b = to_host(B)
+    assert slate_amd.posv(A, B, uplo=uplo) == 0
+    x = to_host(B)
+    scale = np.abs(S).sum(1).max() * np.abs(x).max()
+    assert np.abs(b - S @ x).max() <= 16 * n * np.finfo(np.float64).eps * scale
+
+
+def test_getrs_matrix_extreme_diagonal(gpu):
+    """Diagonal entries whose reciprocal overflows take the dividing branch of
+    the one-launch solve; rows next to them keep full accuracy."""
+    n, nrhs = 64, 8
+    F = np.eye(n)
+    F[5, 5] = 1e-310
+    F[40, 40] = 1e300
+    A = to_dev(F)
+    b = np.ones((n, nrhs))
+    b[5] = 3e-310
+    B = to_dev(b)
+    slate_amd.getrs(A, np.arange(1, n + 1), B)
+    ref = b / np.diag(F)[:, None]
+    np.testing.assert_allclose(to_host(B), ref, rtol=4 * np.finfo(np.float64).eps, atol=0)
