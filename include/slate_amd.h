@@ -295,7 +295,7 @@ int slate_amd_tune_set_nb(slate_amd_context ctx, int kind, int count, const int6
 int64_t slate_amd_tune_get_nb(slate_amd_context ctx, int kind, int64_t n);
 /* Tile configuration of the batched solver: float panel width nbf (16 or
  * 32; the FP64 panel is half as wide), workgroup size bt (256, or 512 with
- * nbf 16) and workgroups per CU (at most what LDS and registers allow, reported in
+ * nbf 16, where two panels are factored as one) and workgroups per CU (at most what LDS and registers allow, reported in
  * max_wgs_per_cu).  Default 32 / 256 / 1 until the autotuner installs its
  * measured choice. */
 int slate_amd_tune_set_batched(slate_amd_context ctx, int nbf, int bt, int wgs_per_cu);

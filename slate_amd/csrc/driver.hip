@@ -2819,7 +2819,6 @@ static int64_t batched_run(sa::Context& c, int count, const int* n, const double
         b += n[i];
         order[i] = i;
     }
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return n[x] > n[y]; });
     // use_graph means the batched launch's own one-node graph here (the LU
     // step-sequence graph that read_opts guards is a different path)
     slate_amd_options oc;
@@ -2828,6 +2827,17 @@ static int64_t batched_run(sa::Context& c, int count, const int* n, const double
     const bool use_graph = oc.use_graph != 0;
     oc.use_graph = 0;
     sa::Opts o = sa::read_opts(&oc);
+    // systems that one wave solves go last, in groups of a workgroup's waves
+    // (fewer per workgroup where that leaves workgroups idle)
+    const bool probe_bf16 = oc.factor_precision == SLATE_AMD_PREC_BF16;
+    auto small = [&](int i) {
+        return n[i] <= sa::batched_small_n() && modes[i] != 2 && !(modes[i] >= 3 && probe_bf16);
+    };
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+        const bool sx = small(x), sy = small(y);
+        return sx != sy ? sy : n[x] > n[y];
+    });
+    const int nbig = int(std::find_if(order.begin(), order.end(), small) - order.begin());
     SA_ENTRY_SYNC();
     sa::Timer t(c);
     // metadata: offA, offB, ticks (8 bytes) | berr (double) | n, mode, order, iters, info, choice (int) |
@@ -2861,13 +2871,15 @@ static int64_t batched_run(sa::Context& c, int count, const int* n, const double
     if (nsel) SA_HIP(hipMemcpyAsync(d_sel, sel, sizeof(float) * nsel, hipMemcpyHostToDevice, c.s0));
     int cus = 0;
     SA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device));
-    const int grid = std::max(1, std::min(count, cus * c.b_wgs));
+    const int wgs = cus * c.b_wgs, nsmall = count - nbig;
+    const int per = nsmall > 0 ? std::max(1, std::min(c.b_bt / 64, (nsmall + wgs - 1) / wgs)) : 0;
+    const int grid = std::max(1, std::min(nbig + (per ? (nsmall + per - 1) / per : 0), wgs));
     c.bwork.ensure(size_t(grid) * size_t(sa::batched_work_stride()));
     alignas(16) char args[sa::BATCH_ARGS_BYTES] = {};
-    sa::batched_fill_args(args, count, d_order, d_n, d_mode, d_offA, d_offB, dA, dB, dX, d_iters, d_info, d_berr,
+    sa::batched_fill_args(args, count, nbig, per, d_order, d_n, d_mode, d_offA, d_offB, dA, dB, dX, d_iters, d_info, d_berr,
                           d_choice, features ? d_feat : nullptr, ms ? d_ticks : nullptr, nsel ? d_sel : nullptr,
                           c.bqueue.as<int>(), static_cast<char*>(c.bwork.p), int(o.itermax), o.tol,
-                          oc.factor_precision == SLATE_AMD_PREC_BF16 ? 1 : 0);
+                          probe_bf16 ? 1 : 0);
     if (use_graph) {
         const int cfg[3] = {c.b_nbf, c.b_bt, grid};
         if (!c.bgraph_exec || memcmp(args, c.bgraph_args, sizeof(args)) != 0

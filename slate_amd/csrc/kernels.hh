@@ -74,9 +74,10 @@ void mlp_train(float* P, float* grad, float* m, float* v, const float* X, const 
 constexpr int BATCH_ARGS_BYTES = 256;
 int64_t batched_work_stride(int elem_bytes = 4);
 int batched_max_n();
+int batched_small_n();                // most rows of a system that one wave solves (not with a BF16 factor)
 bool batched_config_valid(int nbf, int bt);
 int batched_max_wgs_per_cu(int nbf, int bt);
-void batched_fill_args(void* out, int count, const int* order, const int* n, const int* mode, const int64_t* offA,
+void batched_fill_args(void* out, int count, int nbig, int small_per, const int* order, const int* n, const int* mode, const int64_t* offA,
                        const int64_t* offB, const double* A, const double* B, double* X, int* iters, int* info,
                        double* berr, int* choice, float* feat, unsigned long long* ticks, const float* sel,
                        int* queue, char* work, int itermax, double tol, int probe_bf16);

@@ -200,3 +200,67 @@ def test_getrs_matrix_extreme_diagonal(gpu):
     slate_amd.getrs(A, np.arange(1, n + 1), B)
     ref = b / np.diag(F)[:, None]
     np.testing.assert_allclose(to_host(B), ref, rtol=4 * np.finfo(np.float64).eps, atol=0)
+
+
+def _batch(ns, seed, singular=()):
+    rng = np.random.default_rng(seed)
+    mats, rhs = [], []
+    for i, n in enumerate(ns):
+        M = rng.uniform(-1, 1, (n, n)) + 1.2 * np.sqrt(n) * np.eye(n)[rng.permutation(n)]
+        if i in singular:
+            M[:, n // 2] = 0.0
+        mats.append(M)
+        rhs.append(rng.uniform(-1, 1, n))
+    A = torch.from_numpy(np.concatenate([m.T.ravel() for m in mats])).cuda()
+    B = torch.from_numpy(np.concatenate(rhs)).cuda()
+    return mats, rhs, A, B, torch.zeros_like(B)
+
+
+@pytest.mark.parametrize("ns", [[1] * 5, list(range(1, 66)), [64, 65, 63, 1024, 48, 47, 33, 500],
+                                [(7 * i) % 24 + 1 for i in range(2300)], [96, 97, 127, 128, 129, 160]])
+@pytest.mark.parametrize("prec", [slate_amd.PREC_FP32, slate_amd.PREC_FP64])
+def test_batched_wave_and_workgroup_sizes(gpu, ns, prec):
+    """Systems that one wave solves (up to 64 rows), alone, in full groups and
+    beside workgroup systems.  Solutions against numpy's to 1e-11 relative:
+    the condition numbers stay below about 1e4, and the backward errors below
+    the refinement's tolerance, sqrt(n) eps."""
+    say("batched %d systems up to %d, precision %d" % (len(ns), max(ns), prec))
+    mats, rhs, A, B, X = _batch(ns, 5)
+    iters, info, berr = slate_amd.gesv_batched(ns, A, B, X, prec)
+    assert (info == 0).all() and (iters >= 0).all()
+    assert (berr <= np.sqrt(np.asarray(ns)) * np.finfo(np.float64).eps * (1 if prec == slate_amd.PREC_FP32 else 32)).all()
+    x = X.cpu().numpy()
+    o = 0
+    for M, b, n in zip(mats, rhs, ns):
+        ref = np.linalg.solve(M, b)
+        np.testing.assert_allclose(x[o:o + n], ref, rtol=0, atol=1e-11 * np.abs(ref).max())
+        o += n
+
+
+def test_batched_singular_small_and_large(gpu):
+    """A zero column: info names it after the FP64 fallback, iters = -3, and
+    the other systems are solved."""
+    ns = [20, 64, 3, 100, 50]
+    bad = (0, 1, 3)
+    mats, rhs, A, B, X = _batch(ns, 6, bad)
+    iters, info, _ = slate_amd.gesv_batched(ns, A, B, X, slate_amd.PREC_FP32)
+    x = X.cpu().numpy()
+    o = 0
+    for i, (M, b, n) in enumerate(zip(mats, rhs, ns)):
+        if i in bad:
+            assert info[i] == n // 2 + 1 and iters[i] == -3
+        else:
+            assert info[i] == 0 and iters[i] >= 0
+            np.testing.assert_allclose(x[o:o + n], np.linalg.solve(M, b), rtol=0, atol=1e-11)
+        o += n
+
+
+def test_batched_no_iterations(gpu):
+    """max_iterations 0 and -1: only a first solve that already meets the
+    tolerance counts, and none does with -1."""
+    ns = [30, 200]
+    mats, rhs, A, B, X = _batch(ns, 7)
+    for most, want in ((0, -1), (-1, 0)):
+        iters, info, _ = slate_amd.gesv_batched(ns, A, B, X, slate_amd.PREC_FP32,
+                                                opts=slate_amd.Options(max_iterations=most))
+        assert (info == 0).all() and (iters == want).all()
