@@ -136,7 +136,6 @@ void panel_leaf(T* A, int64_t ld, int64_t r0, int64_t m_total, int64_t c0, int w
                 int64_t* ipiv, int64_t* info, double threshold, const PanelWork& pw,
                 uint32_t tag0, hipStream_t s, int64_t xp0 = 0, int64_t xpw = 0);
 int panel_leaf_width(int elem_bytes);   // largest leaf width the kernel supports
-int64_t panel_leaf_wg_rows(int elem_bytes, int W);   // most rows of the one-workgroup form
 
 // Tournament-pivoting leaf (MethodLU::CALU): same contract as panel_leaf
 // with the pivots chosen by a butterfly tournament over the workgroups; uses

@@ -23,9 +23,9 @@ namespace sa {
 // stage and finished rows meet a zero factor (a wave that sees a non-finite
 // factor puts them aside meanwhile).
 // FP64, 32 columns of 100 rows: 140 us per leaf with the exchange through
-// memory (which one workgroup does not need), 50 us here; 1000 rows 146 and
-// 76 us; 16 columns of 2000 rows 46 us, where 32 took 146 us.  A column is
-// about 3000 cycles, of which the two barriers and the LDS round trips
+// memory that one workgroup does not need, 50 us here, and 500 rows as much;
+// with two rows per thread 1000 rows 69 us, where the exchange now takes 64.
+// A column of that is about 3000 cycles, of which the two barriers and the LDS round trips
 // between them are a third.
 template <class T>
 struct LeafEntry { T abs, val, inv; uint32_t idx; };       // a wave's candidate

@@ -4,13 +4,12 @@
 // with partial pivoting.  It replaces SLATE's host panel (internal::getrf_panel
 // <HostTask>, src/internal/internal_getrf.cc:20-121, which pulls the panel to
 // the CPU every step) by a GPU kernel in which G workgroups each keep a slice
-// of rows in registers.  Per column, each workgroup finds its local pivot
-// candidate with wavefront shuffles and publishes it (value, row, and the row's
-// W entries) as tagged words to a double-buffered exchange area; every
-// workgroup reads the G (value, row) heads (one memory round trip once they
-// have landed, with no grid barrier and no fences), reduces them itself,
-// fetches the winning row, applies the interchange to the rows it owns, scales
-// and performs the rank-1 update.
+// of rows in registers.  Per column, each workgroup publishes its pivot
+// candidate as tagged words to a double-buffered exchange area; every
+// workgroup reads the G candidates (one memory round trip once they have
+// landed, with no grid barrier and no fences), picks the winner itself and
+// finishes the next column with it; the rest of the pivot row follows while
+// the next candidates travel.
 // Pivot rules follow src/internal/Tile_getrf.hh:197-366: largest |a_ij| with
 // the smallest row winning exact ties, the diagonal kept when
 // |a_jj| >= threshold * max, scaling by the reciprocal unless the pivot is
@@ -22,53 +21,32 @@
 
 namespace sa {
 
-static constexpr int LEAF_GMAX = 128;     // workgroups per leaf launch
-
 template <class T> struct LeafW;
 template <> struct LeafW<double> { static constexpr int W = 32; };
 template <> struct LeafW<float> { static constexpr int W = 32; };
 
 int panel_leaf_width(int elem_bytes) { return elem_bytes == 8 ? LeafW<double>::W : LeafW<float>::W; }
 
-// Exchange area (64-bit tagged words, see tw_store in common.hh), per column
-// parity: G candidate entries of CW words [|a| (NWV words), row index (1
-// word), the candidate row (W values)], then row j (W values).  NWV = words
-// per value.  Column j of a launch carries tag tag0 + j; alternating parity
-// areas keep a workgroup that runs one column ahead from overwriting words
-// that a slower one has not read yet.
+// Exchange area (64-bit tagged words, see tw_store in common.hh).  Heads, one
+// area per column parity: G + 1 entries of HW words, the candidates and row j
+// (value, factor of the last column, entry of the next column, row index; a
+// value is two words, the low one first, in FP64).  Pivot rows, one area per column parity:
+// REP copies of W values in rotated order, workgroup g reads copy g mod REP
+// (all of them polling one copy would queue up on its few cache lines).
+// Column j of a launch carries tag tag0 + j.  Areas are reused only when every
+// reader is through: a workgroup publishes its head j + 2 after it has read
+// every head j + 1, which the others publish after they have read the heads
+// j; and row j + 2 goes out after every head j + 2, which a workgroup
+// publishes when its waves have read row j.
 template <class T, int W>
 struct LeafSlots {
-    static constexpr int NWV = int(sizeof(T)) / 4;
-    static constexpr int CW = NWV * (W + 1) + 1;
-    static constexpr int MAXWORDS = LEAF_GMAX * CW + W * NWV;
-    __host__ __device__ static int64_t per(int G) { return (int64_t(G) * CW + W * NWV + 63) & ~int64_t(63); }
+    static constexpr int NWV = int(sizeof(T)) / 4;         // words per value
+    static constexpr int HW = 4 * NWV;
+    static constexpr int RW = W * NWV;
+    static constexpr int REP = 8;
+    __host__ __device__ static int64_t heads(int G) { return (int64_t(G) + 1) * HW; }
+    __host__ __device__ static int64_t words(int G) { return 2 * heads(G) + 2 * REP * RW; }
 };
-
-template <class T>
-__device__ inline T lds_val(const uint32_t* w)
-{
-    if constexpr (sizeof(T) == 8) return __builtin_bit_cast(T, (uint64_t(w[1]) << 32) | w[0]);
-    else return __builtin_bit_cast(T, w[0]);
-}
-
-template <class T>
-__device__ inline void lds_put_val(uint32_t* w, T v)
-{
-    if constexpr (sizeof(T) == 8) {
-        const uint64_t u = __builtin_bit_cast(uint64_t, v);
-        w[0] = uint32_t(u);
-        w[1] = uint32_t(u >> 32);
-    }
-    else {
-        w[0] = __builtin_bit_cast(uint32_t, v);
-    }
-}
-
-template <class T>
-__device__ inline bool better(T a, int64_t ia, T b, int64_t ib)
-{
-    return a > b || (a == b && ia < ib);
-}
 
 //------------------------------------------------------------------------------
 // The leaf's w interchanges (row j <-> row piv[j], sequentially, rows local to
@@ -150,275 +128,422 @@ __device__ void leaf_swap_others(T* __restrict__ A, int64_t ld, int64_t r0, int6
 }
 
 //------------------------------------------------------------------------------
-// Leaf with rotated register columns.  v[q][c] holds column (j + c) mod W at
-// step j, so the active column is always v[q][0] and every other access uses
-// compile-time register indices (no per-element column selects); one
-// circular shift per step keeps the invariant.  Rows are published and kept
-// in LDS in the same rotated order.  The exchange is in two stages: every
-// workgroup gathers only the G (|a|, row) heads and row j (G*(NWV+1) + W*NWV
-// words, about one per thread), decides the pivot, and then wave 0 reads the
-// winner's row, which the winner published in the same round (no second read
-// when the diagonal is kept).
-template <class T, int W, int RPT, int VEC, int NT>
-__global__ __launch_bounds__(NT)
-void panel_leaf_rot_kernel(T* __restrict__ A, int64_t ld, int64_t r0, int64_t m_total, int64_t c0,
-                           int w, int64_t* __restrict__ ipiv, int64_t* __restrict__ info, T threshold,
-                           uint32_t tag0, uint64_t* slots, int* error, int64_t xp0, int64_t xpw)
+// A candidate in the form in which it travels, one word per lane: its value,
+// its factor of the column before, its entry of the column after, its row (no
+// candidate: value 0 and the largest row number, which loses to every other).
+template <class T>
+struct alignas(4 * sizeof(T)) LeafHead { T val, fac, nxt; uint32_t idx; };
+// A column's decision: the winner's head and the last pivot row's entry of the
+// column after.
+template <class T>
+struct LeafDec { LeafHead<T> h; T u2; };
+
+__device__ __forceinline__ double fma_of(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fma_of(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
+// Of E candidates in LDS, the largest magnitude, then the smallest row.
+template <class T>
+__device__ __forceinline__ int leaf_best(const LeafHead<T>* h, int E)
+{
+    const int lane = threadIdx.x & 63;
+    T ba = T(-1);
+    uint32_t bi = 0xFFFFFFFFu;
+    int be = 0;
+    for (int e = lane; e < E; e += 64) {
+        const T a = fabs(h[e].val);
+        const uint32_t x = h[e].idx;
+        const bool take = a > ba || (a == ba && x < bi);
+        ba = take ? a : ba;
+        bi = take ? x : bi;
+        be = take ? e : be;
+    }
+    const uint32_t key = argmax_key(ba);
+    const int l = wave_argmax_lane(ba, bi, key, wave_max_u32(key));
+    return __builtin_amdgcn_readlane(be, l);
+}
+
+// The exchange of a leaf, by one wave of each workgroup: per column, between
+// two barriers, it publishes the workgroup's candidate, gathers the heads of
+// all workgroups, 64 words per load, and picks the winner out of its
+// registers.  One wave issues an instruction about every five cycles, so the
+// words stay on the lanes that loaded them: magnitudes order like their
+// leading words, six DPP maxima find the largest, and its lanes store the head
+// on.  Several of the same leading word are compared in LDS (s_tie).
+template <class T, int W, int NW, int GMAX>
+__device__ __forceinline__ void leaf_exchange(int w, int m, int64_t r0, int64_t c0, int64_t* __restrict__ ipiv,
+                                              int64_t* __restrict__ info, T threshold, uint32_t tag0, uint64_t* slots,
+                                              int* error, const LeafHead<T>* s_cand, LeafHead<T>* s_tie,
+                                              LeafDec<T>* s_dec, int* s_pivs)
 {
     using SL = LeafSlots<T, W>;
-    constexpr int NWV = SL::NWV, CW = SL::CW;
-    constexpr int HW = NWV + 1;                 // head words of an entry: |a|, row
-    constexpr int AMAX = LEAF_GMAX * HW + W * NWV;
-    constexpr int NCR = (AMAX + NT - 1) / NT;
-    static_assert((W & (W - 1)) == 0 && W % 4 == 0, "W must be a power of two");
-    typedef T vec4_t __attribute__((ext_vector_type(4)));
-    const int G = gridDim.x;
-    const int g = blockIdx.x;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int64_t m = m_total - r0;
-    constexpr int64_t R = int64_t(NT) * RPT;
-    const int64_t gbase = int64_t(g) * R;
-    const int totalA = G * HW + W * NWV;
-    const int64_t per = SL::per(G);
-
-    constexpr int NW = NT / 64;                 // waves per workgroup
-    __shared__ T s_wabs[NW];
-    __shared__ uint32_t s_widx[NW];
-    __shared__ uint32_t s_pub[2][W * NWV];      // rows being published (candidate, row j)
-    __shared__ uint32_t s_words[AMAX];
-    __shared__ __attribute__((aligned(16))) T s_rowj[W];   // row j, rotated
-    __shared__ __attribute__((aligned(16))) T s_piv[W];    // pivot row, rotated
-    __shared__ __attribute__((aligned(16))) T s_prot[W];   // pivot row, rotated, 0 outside columns j+1 .. w-1
-    __shared__ int64_t s_p;
-    __shared__ int s_pivs[W];                   // local pivot row of each column
-
-    constexpr int VE = 16 / int(sizeof(T));
-    T v[RPT][W];
+    typedef uint32_t __attribute__((may_alias)) word_t;
+    constexpr int NWV = SL::NWV, HW = SL::HW, RW = SL::RW;
+    constexpr int EPL = 64 / HW;                           // entries per load
+    constexpr int NU = GMAX / EPL;
+    constexpr int IDX = 3 * NWV, USED = IDX + 1;
+    constexpr int LEAD = NWV - 1;                          // the leading word of the value
+    const int G = gridDim.x, g = blockIdx.x;
+    const int lane = threadIdx.x & 63, k = lane % HW;
+    // load NU: row j's head on the first lanes, then the words of the last
+    // pivot row that belong to column j + 1, tagged one step earlier; lanes
+    // without a word of their own read another's
+    const bool isu = lane >= HW && lane < HW + NWV;
+    const int ku = k < USED ? k : 0;
+    uint32_t off[NU], mask[NU];
     #pragma unroll
-    for (int q = 0; q < RPT; ++q) {
-        int64_t i = gbase + tid + int64_t(NT) * q;
-        const T* rowp = A + (r0 + (i < m ? i : 0)) * ld + c0;
-        if (VEC && w == W) {
-            #pragma unroll
-            for (int c = 0; c < W; c += VE) {
-                typedef T vec_t __attribute__((ext_vector_type(VE)));
-                vec_t x = *reinterpret_cast<const vec_t*>(rowp + c);
-                #pragma unroll
-                for (int e = 0; e < VE; ++e) v[q][c + e] = (i < m) ? x[e] : T(0);
-            }
-        }
-        else {
-            #pragma unroll
-            for (int c = 0; c < W; ++c)
-                v[q][c] = (i < m && c < w) ? rowp[c] : T(0);
-        }
+    for (int u = 0; u < NU; ++u) {
+        const int e = u * EPL + lane / HW;
+        off[u] = uint32_t((e < G ? e : G) * HW + ku);
+        mask[u] = (e < G && k == LEAD) ? 0x7FFFFFFFu : 0u;
     }
-    const T safe_min = std::numeric_limits<T>::min();
-    constexpr uint32_t NONE = 0xFFFFFFFFu;
-    auto better = [](T a, uint32_t ia, T b, uint32_t ib) { return a > b || (a == b && ia < ib); };
-
+    const uint32_t cmask = (lane / HW < NW && k == LEAD) ? 0x7FFFFFFFu : 0u;
     #pragma unroll 1
     for (int j = 0; j < w; ++j) {
-        uint64_t* buf = slots + (j & 1) * per;
+        uint64_t* const head = slots + (j & 1) * SL::heads(G);
+        const uint64_t* const urow = slots + 2 * SL::heads(G) + (((j + 1) & 1) * SL::REP + (g & (SL::REP - 1))) * RW;
         const uint32_t tag = tag0 + uint32_t(j);
-
-        // (1) local candidate: first row i >= j of maximal |a_ij|
-        T babs = T(-1);
-        uint32_t bidx = NONE;
-        #pragma unroll
-        for (int q = 0; q < RPT; ++q) {
-            const int64_t i = gbase + tid + int64_t(NT) * q;
-            const T a = fabs(v[q][0]);
-            const bool take = i >= j && i < m && a > babs;
-            babs = take ? a : babs;
-            bidx = take ? uint32_t(i) : bidx;
-        }
-        wave_argmax(babs, bidx);
-        if (lane == 0) { s_wabs[wave] = babs; s_widx[wave] = bidx; }
-        __syncthreads();
-        babs = s_wabs[0]; bidx = s_widx[0];
-        #pragma unroll
-        for (int k = 1; k < NW; ++k) {
-            const bool b = better(s_wabs[k], s_widx[k], babs, bidx);
-            babs = b ? s_wabs[k] : babs;
-            bidx = b ? s_widx[k] : bidx;
-        }
-
-        // (2) publish the head (|a|, row) first — it is what every workgroup
-        // polls for — then the candidate row and, from the owner of row j,
-        // row j (rotated order).  A row is copied by its owning thread into
-        // LDS and stored by the lanes of that thread's wave, one word each
-        // (one vector store instead of W single-lane stores).
-        uint64_t* ent = buf + int64_t(g) * CW;
-        if (tid == 0) {
-            tw_store_val<T>(ent, babs, tag);
-            tw_store(ent + NWV, bidx, tag);
-        }
-        const int64_t cl = (bidx != NONE) ? int64_t(bidx) - gbase : -1;
-        const int64_t jl = int64_t(j) - gbase;
-        const int cand_t = (cl >= 0 && cl < R) ? int(cl % NT) : -1;
-        const int rowj_t = (jl >= 0 && jl < R) ? int(jl % NT) : -1;
-        #pragma unroll
-        for (int q = 0; q < RPT; ++q) {
-            if (tid == cand_t && q == int(cl / NT)) {
-                #pragma unroll
-                for (int c = 0; c < W; ++c) lds_put_val<T>(&s_pub[0][c * NWV], v[q][c]);
-            }
-            if (tid == rowj_t && q == int(jl / NT)) {
-                #pragma unroll
-                for (int c = 0; c < W; ++c) lds_put_val<T>(&s_pub[1][c * NWV], v[q][c]);
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-        if (cand_t >= 0 && wave == cand_t / 64 && lane < W * NWV) tw_store(ent + HW + lane, s_pub[0][lane], tag);
-        if (rowj_t >= 0 && wave == rowj_t / 64 && lane < W * NWV)
-            tw_store(buf + int64_t(G) * CW + lane, s_pub[1][lane], tag);
-
-        // (3a) gather the heads of all workgroups and row j
+        __syncthreads();                                   // the waves' candidates
         {
-            int64_t off[NCR];
-            bool val[NCR];
-            uint32_t got[NCR];
-            #pragma unroll
-            for (int u = 0; u < NCR; ++u) {
-                const int e = tid + u * NT;
-                const int ee = e < totalA ? e : totalA - 1;
-                val[u] = e < totalA;
-                off[u] = ee < G * HW ? int64_t(ee / HW) * CW + ee % HW : int64_t(G) * CW + (ee - G * HW);
-            }
-            tw_gather<NCR>(buf, off, val, tag, got, error, 1);
-            #pragma unroll
-            for (int u = 0; u < NCR; ++u) {
-                const int e = tid + u * NT;
-                if (e < totalA) s_words[e] = got[u];
-            }
+            // lane e HW + k holds word k of wave e's candidate
+            const uint32_t x = reinterpret_cast<const word_t*>(s_cand + (lane / HW < NW ? lane / HW : NW - 1))[ku];
+            const uint32_t xj = reinterpret_cast<const word_t*>(s_cand + NW)[ku];
+            const uint32_t key = x & cmask;
+            const uint64_t eq = __builtin_amdgcn_ballot_w64(key == wave_max_u32(key));
+            int b = int(__builtin_ctzll(eq)) / HW;
+            if (eq & (eq - 1)) b = leaf_best(s_cand, NW);
+            if (lane / HW == b && k < USED) tw_store(head + int64_t(g) * HW + k, x, tag);
+            if (__builtin_amdgcn_readlane(int(xj), IDX) == j && lane < USED)
+                tw_store(head + int64_t(G) * HW + lane, xj, tag);
         }
-        __syncthreads();
-        // (3b) decide; wave 0 fetches the winner's row unless the diagonal stays
-        if (wave == 0) {
-            T ba = T(-1);
-            uint32_t bi = NONE;
-            int bg;
-            for (int e = lane; e < G; e += 64) {
-                const T a = lds_word_val<T>(&s_words[e * HW]);
-                const uint32_t x = s_words[e * HW + NWV];
-                const bool b = better(a, x, ba, bi);
-                ba = b ? a : ba;
-                bi = b ? x : bi;
-            }
-            wave_argmax(ba, bi);
-            bg = bi == NONE ? -1 : int(int64_t(bi) / R);     // workgroup g owns rows [g R, (g + 1) R)
-            const int lc = lane < W ? lane : 0;
-            const T rj = lds_word_val<T>(&s_words[G * HW + lc * NWV]);
-            const T ajj = lds_word_val<T>(&s_words[G * HW]);
-            // Tile_getrf.hh:283-289: keep the diagonal if it is large enough.
-            const bool diag = bg < 0 || bg >= G || fabs(ajj) >= threshold * ba;
-            int64_t p = diag ? int64_t(j) : int64_t(bi);
-            if (p < j || p >= m) p = j;            // never trust a row outside the leaf
-            T pr = rj;
-            if (p != j) {
-                // the winner's row (published with its head)
-                int64_t off[1] = {int64_t(bg) * CW + HW + (lane < W * NWV ? lane : 0)};
-                bool val[1] = {lane < W * NWV};
-                uint32_t got[1];
-                tw_gather<1>(buf, off, val, tag, got, error, 1);
-                if (lane < W * NWV) s_words[lane] = got[0];   // the heads are consumed
-                __builtin_amdgcn_wave_barrier();
-                pr = lds_word_val<T>(&s_words[lc * NWV]);
-            }
-            if (lane < W) {
-                s_rowj[lane] = rj;
-                s_piv[lane] = pr;
-                s_prot[lane] = (lane >= 1 && lane < w - j) ? pr : T(0);
-            }
-            if (lane == 0) s_p = p;
-        }
-        __syncthreads();
-        const int64_t p = s_p;
-        if (tid == 0) s_pivs[j] = int(p);
-
-        // (4) interchange rows j and p among the rows this thread owns
-        #pragma unroll
-        for (int q = 0; q < RPT; ++q) {
-            const int64_t i = gbase + tid + int64_t(NT) * q;
-            if (i == j) {
+        uint32_t got[NU + 1];
+        {
+            const bool wantu = isu && j > 0 && j + 1 < w;
+            const uint64_t* const px = wantu ? urow + 2 * NWV + (lane - HW) : head + int64_t(G) * HW + ku;
+            const uint32_t tagx = wantu ? tag - 1 : tag;
+            uint64_t t0 = 0;
+            bool first = true;
+            while (true) {
+                uint64_t x[NU + 1];
                 #pragma unroll
-                for (int c = 0; c < W; c += 4) {
-                    const vec4_t x = *reinterpret_cast<const vec4_t*>(&s_piv[c]);
-                    v[q][c] = x[0]; v[q][c + 1] = x[1]; v[q][c + 2] = x[2]; v[q][c + 3] = x[3];
+                for (int u = 0; u < NU; ++u) x[u] = tw_load(head + off[u]);
+                x[NU] = tw_load(px);
+                const int err = __hip_atomic_load(error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                uint32_t bad = uint32_t(x[NU] >> 32) ^ tagx;
+                got[NU] = uint32_t(x[NU]);
+                #pragma unroll
+                for (int u = 0; u < NU; ++u) {
+                    bad |= uint32_t(x[u] >> 32) ^ tag;
+                    got[u] = uint32_t(x[u]);
                 }
-            }
-            else if (i == p) {
-                #pragma unroll
-                for (int c = 0; c < W; c += 4) {
-                    const vec4_t x = *reinterpret_cast<const vec4_t*>(&s_rowj[c]);
-                    v[q][c] = x[0]; v[q][c + 1] = x[1]; v[q][c + 2] = x[2]; v[q][c + 3] = x[3];
+                if (__builtin_amdgcn_ballot_w64(bad != 0) == 0 || err != 0) break;
+                if (first) { t0 = wall_clock64(); first = false; }
+                else if (wall_clock64() - t0 > 400000000ull) {
+                    __hip_atomic_store(error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    break;
                 }
             }
         }
-        const T pv = s_piv[0];
-        if (g == 0 && tid == 0) {
-            ipiv[c0 + j] = r0 + p;
-            if (pv == T(0) && *info == 0) *info = c0 + j + 1;
-        }
-        // (5) scale the column below the pivot and update columns j+1 .. w-1
-        // (rotated 1 .. w-j-1; the others see a zero in s_prot and are kept
-        // by the select, so finished columns stay bit-identical)
-        const bool tiny = fabs(pv) < safe_min;
-        const T inv = T(1) / pv;
-        const int lim = w - j;
+        uint32_t km = 0;
         #pragma unroll
-        for (int q = 0; q < RPT; ++q) {
-            const int64_t i = gbase + tid + int64_t(NT) * q;
-            if (i > j && i < m) {
-                T l = v[q][0];
-                if (pv != T(0)) l = tiny ? l / pv : l * inv;
-                v[q][0] = l;
-                #pragma unroll
-                for (int c = 0; c < W; c += 4) {
-                    const vec4_t x = *reinterpret_cast<const vec4_t*>(&s_prot[c]);
-                    #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (c + e >= 1) v[q][c + e] = (c + e < lim) ? v[q][c + e] - l * x[e] : v[q][c + e];
-                }
-            }
+        for (int u = 0; u < NU; ++u) {
+            const uint32_t key = got[u] & mask[u];
+            km = key > km ? key : km;
         }
-        // (6) rotate: column j + 1 becomes v[q][0]
+        km = wave_max_u32(km);
+        uint32_t bw = got[NU];                             // the winner's words, on lanes bl ...
+        uint64_t any = 0, twice = 0;
         #pragma unroll
-        for (int q = 0; q < RPT; ++q) {
-            const T t0 = v[q][0];
+        for (int u = 0; u < NU; ++u) {
+            const uint64_t eq = __builtin_amdgcn_ballot_w64((got[u] & mask[u]) == km);
+            twice |= any & eq;
+            any |= eq;
+            bw = eq ? got[u] : bw;
+        }
+        int bl = __builtin_ctzll(any) & ~(HW - 1);
+        if (twice | (any & (any - 1))) {
             #pragma unroll
-            for (int c = 0; c < W - 1; ++c) v[q][c] = v[q][c + 1];
-            v[q][W - 1] = t0;
+            for (int u = 0; u < NU; ++u) reinterpret_cast<word_t*>(s_tie)[u * 64 + lane] = got[u];
+            __builtin_amdgcn_wave_barrier();
+            bw = reinterpret_cast<const word_t*>(s_tie + leaf_best(s_tie, G))[ku];
+            bl = 0;
+            __builtin_amdgcn_wave_barrier();
+        }
+        // Tile_getrf.hh:283-289: keep the diagonal if it is large enough (a
+        // threshold of 1 keeps it where it is the first of the largest, the
+        // winner); never take a row outside the leaf
+        const uint32_t bi = uint32_t(__builtin_amdgcn_readlane(int(bw), bl + IDX));
+        bool keep = bi < uint32_t(j) || bi >= uint32_t(m);
+        if (threshold < T(1)) {
+            if (lane / HW == bl / HW) reinterpret_cast<word_t*>(s_tie)[k] = bw;
+            if (lane < HW) reinterpret_cast<word_t*>(s_tie + 1)[k] = got[NU];
+            __builtin_amdgcn_wave_barrier();
+            keep = keep || fabs(s_tie[1].val) >= threshold * fabs(s_tie[0].val);
+            keep = __builtin_amdgcn_ballot_w64(keep) != 0;
+            __builtin_amdgcn_wave_barrier();
+        }
+        bw = keep ? (k == IDX ? uint32_t(j) : got[NU]) : bw;
+        bl = keep ? 0 : bl;
+        if (lane / HW == bl / HW && k < USED) reinterpret_cast<word_t*>(&s_dec->h)[k] = bw;
+        if (isu) reinterpret_cast<word_t*>(&s_dec->u2)[lane - HW] = got[NU];
+        if (lane == bl + IDX) s_pivs[j] = int(bw);
+        __syncthreads();                                   // the decision
+        if (g == 0) {
+            if (lane == bl + IDX) ipiv[c0 + j] = r0 + int64_t(bw);
+            if (lane == 0 && s_dec->h.val == T(0) && *info == 0) *info = c0 + j + 1;
         }
     }
+}
 
-    // after w steps v[q][c] holds column (w + c) mod W
-    #pragma unroll
-    for (int q = 0; q < RPT; ++q) {
-        int64_t i = gbase + tid + int64_t(NT) * q;
-        if (i < m) {
-            T* rowp = A + (r0 + i) * ld + c0;
-            if (VEC && w == W) {
+// Leaf over G workgroups of NT / 64 waves with rows and one for the exchange.
+// v[q][c] of a thread holds column (j + c) mod W of its q-th row at step j, so
+// every register index is a constant; rows never move, an interchange swaps
+// their labels, and a row is stored at its label.
+// Bound: the exchange between workgroups, one publication and one read per
+// column, so little else stays on that chain:
+//  - The pivot row travels beside it.  A head carries the candidate's value,
+//    its factor l of the column before, and its entry of the column after as
+//    it was before that column's update; with the pivot row of the column
+//    before, which has arrived by then, every workgroup forms the one entry
+//    u1 = next - l u that the next search needs, by the operation that the
+//    row's owner applies.  The other entries are read and used while the next
+//    heads travel.
+//  - The exchanging wave has no rows, so updates and exchange overlap.
+// Us per column, before (heads, then the row, then everything) and now: FP64,
+// 8192 rows 4.6 and 2.3; FP32, 16384 rows 5.1 and 2.4, 65536 rows 7.1 and 2.8.
+// Of 4900 cycles (FP64, 8192 rows) the heads' way through memory is 2300, the
+// search 700, picking the winner 700, scaling 570, publishing 500; the pivot
+// row arrives 2700 cycles after its column's search.
+template <class T, int W, int RPT, int NT, int GMAX>
+__global__ __launch_bounds__(NT + 64, RPT * W * sizeof(T) <= 256 ? 4 : 1)
+void panel_leaf_rot_kernel(T* __restrict__ A, int64_t ld, int64_t r0, int64_t m_total, int64_t c0,
+                           int w, int64_t* __restrict__ ipiv, int64_t* __restrict__ info, T threshold,
+                           uint32_t tag0, uint64_t* slots, int* error, int64_t xp0, int64_t xpw, bool vec)
+{
+    using SL = LeafSlots<T, W>;
+    constexpr int NWV = SL::NWV, RW = SL::RW;
+    constexpr int NW = NT / 64;
+    constexpr int VE = 16 / int(sizeof(T));
+    constexpr uint32_t NONE = 0xFFFFFFFFu;
+    static_assert((W & (W - 1)) == 0 && RW <= 64 && W % VE == 0, "a row is one word per lane");
+    static_assert(NW <= 8, "one candidate per lane of a group of eight");
+    typedef T vec_t __attribute__((ext_vector_type(VE)));
+    typedef uint32_t __attribute__((may_alias)) word_t;
+    const int G = gridDim.x;
+    const int g = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m = int(m_total - r0);
+    const T safe_min = std::numeric_limits<T>::min();
+
+    __shared__ LeafHead<T> s_cand[NW + 1];                     // the waves', and row j if it is here
+    __shared__ LeafHead<T> s_tie[GMAX];
+    __shared__ LeafDec<T> s_dec;
+    __shared__ __attribute__((aligned(16))) T s_row[NW][W];    // each wave's copy of the pivot row
+    __shared__ T s_raw[NW][W];                                 // the same with what is not finite
+    __shared__ int s_pivs[W];                                  // local pivot row of each column
+
+    if (wave == NW) {
+        if (lane == 0) s_cand[NW].idx = NONE;                  // before the first barrier
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    if (wave == NW) {
+        leaf_exchange<T, W, NW, GMAX>(w, m, r0, c0, ipiv, info, threshold, tag0, slots, error, s_cand, s_tie,
+                                      &s_dec, s_pivs);
+    }
+    else {
+        const int gbase = g * NT * RPT;
+        uint64_t* const rows = slots + 2 * SL::heads(G);
+        // in the order of step -1: column c at position c + 1
+        T v[RPT][W], nxt[RPT], l[RPT];
+        int lab[RPT];                                          // the row each register row stands for
+        #pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+            const int i = gbase + tid + NT * q;
+            lab[q] = i;
+            const T* rowp = A + (r0 + (i < m ? i : 0)) * ld + c0;
+            if (vec) {
                 #pragma unroll
                 for (int c = 0; c < W; c += VE) {
-                    typedef T vec_t __attribute__((ext_vector_type(VE)));
-                    vec_t x;
+                    const vec_t x = *reinterpret_cast<const vec_t*>(rowp + c);
                     #pragma unroll
-                    for (int e = 0; e < VE; ++e) x[e] = v[q][c + e];
-                    *reinterpret_cast<vec_t*>(rowp + c) = x;
+                    for (int e = 0; e < VE; ++e) v[q][(c + e + 1) % W] = x[e];
                 }
             }
             else {
                 #pragma unroll
-                for (int c = 0; c < W; ++c) {
-                    const int col = (w + c) & (W - 1);
-                    if (col < w) rowp[col] = v[q][c];
+                for (int c = 0; c < W; ++c) v[q][(c + 1) % W] = rowp[c < w ? c : 0];
+            }
+            #pragma unroll
+            for (int c = 0; c < W; ++c) v[q][(c + 1) % W] = (i < m && c < w) ? v[q][(c + 1) % W] : T(0);
+            nxt[q] = v[q][1];
+            l[q] = T(0);
+        }
+        int pl = -1, pq = 0;                                   // the last pivot row's lane in this wave
+
+        #pragma unroll 1
+        for (int j = 0; j < w; ++j) {
+            const uint32_t tag = tag0 + uint32_t(j);
+            // (1) this wave's candidate: the largest entry of column j, the first of equals
+            T babs = T(-1), bval = T(0), bfac = T(0), bnxt = T(0);
+            uint32_t bidx = NONE;
+            #pragma unroll
+            for (int q = 0; q < RPT; ++q) {
+                const T a = fabs(nxt[q]);
+                const bool take = lab[q] >= j && lab[q] < m && (a > babs || (a == babs && uint32_t(lab[q]) < bidx));
+                babs = take ? a : babs;
+                bval = take ? nxt[q] : bval;
+                bfac = take ? l[q] : bfac;
+                bnxt = take ? v[q][2] : bnxt;
+                bidx = take ? uint32_t(lab[q]) : bidx;
+                if (lab[q] == j) s_cand[NW] = LeafHead<T>{nxt[q], l[q], v[q][2], uint32_t(j)};
+            }
+            const uint32_t key = argmax_key(babs);
+            const uint32_t mk = wave_max_u32(key);
+            const int wl = wave_argmax_lane(babs, bidx, key, mk);
+            if (lane == wl) s_cand[wave] = LeafHead<T>{bval, bfac, bnxt, bidx};
+            __syncthreads();
+            // (2) the pivot row of column j - 1 goes out ...
+            uint64_t* const rowb = rows + ((j + 1) & 1) * SL::REP * RW;
+            if (pl >= 0) {
+                #pragma unroll
+                for (int q = 0; q < RPT; ++q)
+                    if (q == pq && lane == pl) {
+                        #pragma unroll
+                        for (int c = 0; c < W; c += VE) {
+                            vec_t x;
+                            #pragma unroll
+                            for (int e = 0; e < VE; ++e) x[e] = v[q][c + e];
+                            *reinterpret_cast<vec_t*>(&s_row[wave][c]) = x;
+                        }
+                    }
+                __builtin_amdgcn_wave_barrier();
+                if (lane < (w - j + 1) * NWV && lane < RW) {
+                    const uint32_t x = reinterpret_cast<const word_t*>(s_row[wave])[lane];
+                    #pragma unroll
+                    for (int r = 0; r < SL::REP; ++r) tw_store(rowb + r * RW + lane, x, tag - 1);
+                }
+            }
+            // ... and comes in; finished columns are zero in it
+            const int lim = w - j + 1;                         // positions lim .. of step j - 1 are finished
+            uint32_t fv;
+            if (pl < 0 && j > 0) {
+                const int64_t off[1] = {lane < RW ? lane : 0};
+                const bool val[1] = {lane < lim * NWV && lane >= NWV && lane < RW};
+                uint32_t got[1];
+                tw_gather<1>(rowb + (g & (SL::REP - 1)) * RW, off, val, tag - 1, got, error, 1);
+                fv = got[0];
+            }
+            else {
+                fv = reinterpret_cast<const word_t*>(s_row[wave])[lane < RW ? lane : 0];
+            }
+            const bool in = j > 0 && lane >= NWV && lane < lim * NWV && lane < RW;
+            if (lane < RW) reinterpret_cast<word_t*>(s_row[wave])[lane] = in ? fv : 0u;
+            // 0 * inf would reach finished rows and columns: what is not finite
+            // is left out of the update and follows by itself
+            constexpr uint32_t EXP = sizeof(T) == 8 ? 0x7FF00000u : 0x7F800000u;
+            bool odd = in && lane % NWV == NWV - 1 && (fv & EXP) == EXP;
+            T lz[RPT];
+            #pragma unroll
+            for (int q = 0; q < RPT; ++q) {
+                const bool act = j > 0 && lab[q] >= j && lab[q] < m, fin = isfinite(l[q]);
+                lz[q] = act && fin ? l[q] : T(0);
+                odd = odd || (act && !fin);
+            }
+            const bool sel = __builtin_amdgcn_ballot_w64(odd) != 0;
+            if (sel) {
+                if (lane < W) {
+                    const T x = s_row[wave][lane];
+                    s_raw[wave][lane] = x;
+                    if (!isfinite(x)) s_row[wave][lane] = T(0);
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+            // (3) update, and move down by one
+            {
+                T v0[RPT];
+                #pragma unroll
+                for (int q = 0; q < RPT; ++q) {
+                    v0[q] = v[q][0];
+                    v[q][0] = nxt[q];
+                }
+                #pragma unroll
+                for (int c = 0; c < W; c += VE) {
+                    const vec_t x = *reinterpret_cast<const vec_t*>(&s_row[wave][c]);
+                    #pragma unroll
+                    for (int e = 0; e < VE; ++e)
+                        if (c + e >= 2)
+                            #pragma unroll
+                            for (int q = 0; q < RPT; ++q) v[q][c + e - 1] = fma_of(-lz[q], x[e], v[q][c + e]);
+                }
+                #pragma unroll
+                for (int q = 0; q < RPT; ++q) v[q][W - 1] = v0[q];
+                if (sel) {
+                    #pragma unroll
+                    for (int c = 2; c < W; ++c) {
+                        const T x = s_raw[wave][c];
+                        #pragma unroll
+                        for (int q = 0; q < RPT; ++q) {
+                            const bool act = j > 0 && lab[q] >= j && lab[q] < m && c < lim;
+                            if (act && (!isfinite(x) || !isfinite(l[q]))) v[q][c - 1] = fma_of(-l[q], x, v[q][c - 1]);
+                        }
+                    }
+                }
+                // before the barrier, not on the chain behind it
+                #pragma unroll
+                for (int q = 0; q < RPT; ++q)
+                    #pragma unroll
+                    for (int c = 0; c < W; ++c) asm volatile("" : "+v"(v[q][c]));
+            }
+            __syncthreads();
+            // (4) interchange rows j and p, scale column j and finish column j + 1
+            const LeafDec<T> d = s_dec;
+            const int p = __builtin_amdgcn_readfirstlane(int(d.h.idx));
+            const T pv = d.h.val;
+            const T u1 = j > 0 ? fma_of(-d.h.fac, d.u2, d.h.nxt) : d.h.nxt;
+            const bool zero = pv == T(0), tiny = fabs(pv) < safe_min;
+            const T inv = T(1) / pv;
+            pl = -1;
+            #pragma unroll
+            for (int q = 0; q < RPT; ++q) {
+                const int lb = lab[q];
+                const uint64_t own = __builtin_amdgcn_ballot_w64(lb == p);
+                if (own) { pl = __builtin_ctzll(own); pq = q; }
+                lab[q] = lb == p ? j : (lb == j ? p : lb);
+                const bool act = lab[q] > j && lab[q] < m;
+                T t = v[q][0] * inv;
+                if (zero || tiny) t = zero ? v[q][0] : v[q][0] / pv;
+                l[q] = t;
+                v[q][0] = act ? t : v[q][0];
+                nxt[q] = (act && j + 1 < w) ? fma_of(-t, u1, v[q][1]) : v[q][1];
+            }
+        }
+
+        // after w steps v[q][c] holds column (w - 1 + c) mod W
+        #pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+            const int i = lab[q];
+            if (i < m) {
+                T* rowp = A + (r0 + i) * ld + c0;
+                if (vec) {
+                    #pragma unroll
+                    for (int c = 0; c < W; c += VE) {
+                        vec_t x;
+                        #pragma unroll
+                        for (int e = 0; e < VE; ++e) x[e] = v[q][(c + e + 1) % W];
+                        *reinterpret_cast<vec_t*>(rowp + c) = x;
+                    }
+                }
+                else {
+                    #pragma unroll
+                    for (int c = 0; c < W; ++c) {
+                        const int col = (w - 1 + c) & (W - 1);
+                        if (col < w) rowp[col] = v[q][c];
+                    }
                 }
             }
         }
     }
-    if (xpw > w) leaf_swap_others<T, W, NT>(A, ld, r0, c0, w, xp0, xpw, s_pivs, G, g);
+    if (xpw > w) leaf_swap_others<T, W, NT + 64>(A, ld, r0, c0, w, xp0, xpw, s_pivs, G, g);
 }
 
 //------------------------------------------------------------------------------
@@ -487,25 +612,11 @@ void panel_leaf_wg_kernel(T* __restrict__ A, int64_t ld, int64_t r0, int64_t m_t
     if (xpw > w) leaf_swap_others<T, W, NT, 64>(A, ld, r0, c0, w, xp0, xpw, s.pivs, 1, 0);
 }
 
-// Leaf shape (NT threads, RPT rows each).  Measured per column: FP32 W = 32
-// at m = 65536: 256 x 4 7.8 us, 512 x 2 7.1 us, 1024 x 1 7.5 us, 1024 x 2
-// 22.7 us; at m = 16384: 256 x 1 (G = 64) 5.8 us, 512 x 1 (G = 32) 5.1 us;
-// at m = 8192: 256 x 1 (G = 32) 4.8 us.  Fewer, fatter workgroups lose
-// more in their own barriers and updates than they save in gathered heads,
-// and a one-round gather of every candidate row (no second read of the
-// winner's row) measured no faster at G <= 16 (m = 8192, 512 x 1: 5.1 us).
-static void leaf_shape(int64_t m, int& nt, int& rpt)
-{
-    if (m <= 32 * 256) { nt = 256; rpt = 1; }
-    else if (m <= 64 * 512) { nt = 512; rpt = 1; }
-    else { nt = 512; rpt = 2; }
-}
-
-// Most rows of a one-workgroup leaf of width W: 512 threads keep 4 rows of 128
-// bytes each in registers, or 2 of 256 (190 - 217 registers; more rows spill,
-// and one CU then also spends longer loading and storing the block than the
-// exchange takes).
-int64_t panel_leaf_wg_rows(int elem_bytes, int W) { return W * elem_bytes <= 128 ? 2048 : 1024; }
+// Most rows of a one-workgroup leaf, one row per thread.  FP64, 32 columns:
+// 500 rows 50 us in one workgroup, 63 us over two; 700 rows (two per thread)
+// 64 and 62 us, 1000 rows 69 and 64 us.  FP32: 500 rows 42 and 52 us, 1000
+// rows 53 and 54 us, 2000 rows 78 and 61 us.
+static constexpr int64_t LEAF_WG_ROWS = 512;
 
 template <class T, int W>
 static void panel_leaf_w(T* A, int64_t ld, int64_t r0, int64_t m_total, int64_t c0, int w,
@@ -542,34 +653,41 @@ static void panel_leaf_w(T* A, int64_t ld, int64_t r0, int64_t m_total, int64_t 
     const bool vec = (reinterpret_cast<uintptr_t>(A) % 16 == 0) && (ld % VE == 0) && (c0 % VE == 0);
     SA_REQUIRE(xpw == 0 || (r0 == c0 && xp0 <= c0 && c0 + w <= xp0 + xpw), -2,
                "panel_leaf: leaf outside the enclosing panel");
-#define SA_WG(NTV, R, V) hipLaunchKernelGGL((panel_leaf_wg_kernel<T, W, R, V, NTV>), dim3(1), dim3(NTV), 0, s, \
-                                             A, ld, r0, m_total, c0, w, ipiv, info, thr, xp0, xpw)
-#define SA_WG_V(NTV, R) do { if (vec) SA_WG(NTV, R, 1); else SA_WG(NTV, R, 0); } while (0)
-    if (m <= panel_leaf_wg_rows(int(sizeof(T)), W)) {
-        if (m <= 256) SA_WG_V(256, 1);
-        else if (m <= 512) SA_WG_V(512, 1);
-        else if (m <= 1024) SA_WG_V(512, 2);
-        else if constexpr (W * sizeof(T) <= 128) SA_WG_V(512, 4);
+    if (m <= LEAF_WG_ROWS) {
+#define SA_WG(NTV, V) hipLaunchKernelGGL((panel_leaf_wg_kernel<T, W, 1, V, NTV>), dim3(1), dim3(NTV), 0, s, \
+                                          A, ld, r0, m_total, c0, w, ipiv, info, thr, xp0, xpw)
+        if (m <= 256) { if (vec) SA_WG(256, 1); else SA_WG(256, 0); }
+        else { if (vec) SA_WG(512, 1); else SA_WG(512, 0); }
+#undef SA_WG
         SA_CHECK_LAUNCH();
         return;
     }
-#undef SA_WG_V
-#undef SA_WG
-    int nt = 256, rpt = 1;
-    leaf_shape(m, nt, rpt);
-    int64_t G = ceildiv(m, int64_t(nt) * rpt);
-    SA_REQUIRE(G <= LEAF_GMAX, -2, "panel_leaf: panel too tall");
-    const int64_t slot_bytes = int64_t(2 * sizeof(uint64_t)) * LeafSlots<T, W>::per(int(G));
-    SA_REQUIRE(slot_bytes <= pw.slots_bytes, -2, "panel_leaf: slot area too small");
     uint64_t* slots = static_cast<uint64_t*>(pw.slots);
-#define SA_LEAF(NTV, R, V) hipLaunchKernelGGL((panel_leaf_rot_kernel<T, W, R, V, NTV>), dim3(G), dim3(NTV), 0, s, \
-                                               A, ld, r0, m_total, c0, w, ipiv, info, thr, tag0, slots, pw.error, \
-                                               xp0, xpw)
-#define SA_LEAF_V(NTV, R) do { if (vec) SA_LEAF(NTV, R, 1); else SA_LEAF(NTV, R, 0); } while (0)
-    if (nt == 256) SA_LEAF_V(256, 1);
-    else if (rpt == 1) SA_LEAF_V(512, 1);
-    else SA_LEAF_V(512, 2);
-#undef SA_LEAF_V
+    const bool vec_rows = vec && w == W;
+#define SA_LEAF(NTV, R, GM)                                                                       \
+    do {                                                                                          \
+        const int64_t G = ceildiv(m, int64_t(NTV) * (R));                                         \
+        SA_REQUIRE(G <= (GM), -2, "panel_leaf: panel too tall");                                  \
+        SA_REQUIRE((int64_t(sizeof(uint64_t)) * LeafSlots<T, W>::words(int(G)) <= pw.slots_bytes), -2, \
+                   "panel_leaf: slot area too small");                                            \
+        hipLaunchKernelGGL((panel_leaf_rot_kernel<T, W, R, NTV, GM>), dim3(G), dim3(NTV + 64), 0, s, A, ld, r0, \
+                           m_total, c0, w, ipiv, info, thr, tag0, slots, pw.error, xp0, xpw, vec_rows); \
+    } while (0)
+    // Alone, more workgroups of one row per thread are fastest (FP64, 8192
+    // rows: 256 x 1 2.34 us per column, 256 x 2 2.97).  Beside a trailing
+    // update a leaf starts when enough CUs have retired a GEMM workgroup, and
+    // 8 waves of at most 128 registers fit the place of one (256 registers on
+    // each SIMD): with 256 x 1, 128 workgroups, a leaf of 32768 rows took 935
+    // us beside the FP64 update and 89 alone, with 448 x 1, 74 workgroups, 379
+    // (n = 32768: 660 and 490 ms).  Two rows of 128 bytes fit those registers,
+    // two of 256 do not.  The heads of 32, 64 or 128 workgroups are 4, 8 or 16
+    // loads per poll in FP64 (8192 rows: 2.34, 2.45, 2.72 us), half in FP32.
+    if (m <= 32 * 256) SA_LEAF(256, 1, 32);
+    else if (m <= 64 * 448) SA_LEAF(448, 1, 64);
+    else if (W * sizeof(T) > 128 && m <= 128 * 448) SA_LEAF(448, 1, 128);
+    else if (W * sizeof(T) <= 128 && m <= 64 * 896) SA_LEAF(448, 2, 64);
+    else if (m <= 128 * 896) SA_LEAF(448, 2, 128);
+    else SA_LEAF(512, 2, 128);
 #undef SA_LEAF
     SA_CHECK_LAUNCH();
 }

@@ -1,7 +1,8 @@
-"""GPU tests of the one-workgroup leaf kernels at the edges of their ranges:
+"""GPU tests of the leaf kernels at the edges of their ranges:
 the Cholesky leaf (64 x 64, four register stages of 16 rows) and the inverted
 diagonal blocks of the look-back solves (64 rows FP64, 128 rows FP32, four
-stages), and the LU panel leaf (one workgroup up to 1024 or 2048 rows)."""
+stages), and the LU panel leaf (one workgroup up to 512 rows, an exchange of up
+to 128 above)."""
 import numpy as np
 import pytest
 import torch
@@ -123,6 +124,76 @@ def test_panel_leaf_non_finite(gpu, value, n):
 
 # 32 x 64 tiles (few tiles), 64 x 64 and 128 x 128 tiles, each with whole
 # tiles, ragged edges, a k tail, and operands one element off 16-byte alignment
+@pytest.mark.parametrize("n,dtype", [(520, torch.float64), (8321, torch.float64), (28801, torch.float64),
+                                     (8321, torch.float32), (28801, torch.float32)])
+def test_panel_leaf_exchange_shapes(gpu, n, dtype):
+    """Leaf shapes of several workgroups: every panel of the factorization is
+    pivoted strictly (|L| <= 1) and P A = L U within n eps |L| |U| for the
+    factorization and as much for the product that checks it."""
+    say("panel leaf exchange n=%d %s" % (n, dtype))
+    g = torch.Generator("cuda").manual_seed(n)
+    A = torch.empty(n, n, dtype=dtype, device="cuda").uniform_(-1, 1, generator=g).t()
+    F = A.t().clone().t()
+    info, ipiv = slate_amd.getrf(F)
+    assert info == 0
+    perm = np.arange(n)
+    for i, p in enumerate(ipiv):
+        perm[i], perm[p - 1] = perm[p - 1], perm[i]
+    rows = torch.from_numpy(np.r_[0:200, n // 2:n // 2 + 100, n - 200:n]).cuda()
+    L = torch.where(rows[:, None] > torch.arange(n, device="cuda")[None, :], F[rows], 0)
+    assert float(L.abs().max()) <= 1.0
+    L[torch.arange(len(rows), device="cuda"), rows] = 1.0
+    U = F.triu()
+    PA = A[torch.from_numpy(perm).cuda()[rows]]
+    bound = 2 * n * torch.finfo(dtype).eps * (L.abs() @ U.abs())
+    assert bool(((PA - L @ U).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("n", [512, 1024, 2048])
+def test_panel_leaf_ties(gpu, n):
+    """A Hadamard matrix is eliminated exactly in powers of two and every
+    pivot search is a tie: the first of equals wins, across waves and
+    workgroups, and the factors are the oracle's bit by bit."""
+    say("panel leaf ties n=%d" % n)
+    H = np.array([[1.0]])
+    while H.shape[0] < n:
+        H = np.block([[H, H], [H, -H]])
+    H = np.asfortranarray(H[np.random.default_rng(n).permutation(n)])
+    A = to_dev(H)
+    info, ipiv = slate_amd.getrf(A)
+    LU_o, ipiv_o, info_o = oracle.getrf(H, nb=128, ib=16)
+    assert info == info_o == 0
+    np.testing.assert_array_equal(ipiv, ipiv_o)
+    np.testing.assert_array_equal(to_host(A), LU_o)
+
+
+@pytest.mark.parametrize("n", [300, 700, 1500])
+def test_panel_leaf_threshold(gpu, n):
+    """A pivot threshold keeps diagonals; the oracle's pivots, and its factors
+    within the accumulated rounding (growth is in max |LU|)."""
+    say("panel leaf threshold n=%d" % n)
+    A = dev_rands(77, n, n)
+    info, ipiv = slate_amd.getrf(A, slate_amd.Options(pivot_threshold=0.5, block_size=128))
+    LU_o, ipiv_o, _ = oracle.getrf(oracle.rands(77, n, n), nb=128, ib=16, threshold=0.5)
+    assert info == 0
+    np.testing.assert_array_equal(ipiv[:64], ipiv_o[:64])
+    a, b = to_host(A)[:, :64], LU_o[:, :64]
+    if np.array_equal(ipiv, ipiv_o):
+        assert np.abs(a - b).max() <= 4 * n * np.finfo(np.float64).eps * np.abs(LU_o).max()
+
+
+def test_panel_leaf_zero_column(gpu):
+    """No candidate but zeros in a column of several workgroups: the diagonal
+    stays and info names the column."""
+    say("panel leaf zero column")
+    n = 1500
+    H = oracle.rands(91, n, n).copy(order="F")
+    H[:, 40] = 0.0
+    A = to_dev(H)
+    info, ipiv = slate_amd.getrf(A)
+    assert info == 41 and ipiv[40] == 41
+
+
 @pytest.mark.parametrize("m,n,k", [(70, 130, 200), (64, 128, 128), (1100, 1000, 70), (1088, 1024, 64),
                                    (2100, 2050, 33), (2048, 2176, 48)])
 @pytest.mark.parametrize("off", [0, 1])
