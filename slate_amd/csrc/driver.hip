@@ -1027,36 +1027,31 @@ static T* dinv_pair(Context& c, int64_t n)
     return c.dinv.as<T>();
 }
 
-// Most right-hand sides solved one by one with the look-back sweeps: each
-// costs a read of the factors, the blocked solve a fixed chain of launches.
-constexpr int64_t VEC_RHS_MAX = 4;
-
-// Few right-hand sides: X := op(LU)^{-1} X column by column (ldx apart, each
-// contiguous), using the one-launch look-back triangular solves; tmp holds n.
-// perm is the getrf permutation.
+// Single right-hand side: x := op(LU)^{-1} x with x contiguous, using the
+// one-launch look-back triangular solves.  perm is the getrf permutation.
+// Only one: the sweeps multiply by computed inverses of the diagonal blocks,
+// so their error carries a block's condition, where the blocked solve of
+// several right-hand sides substitutes.
 template <class T>
 static void getrs_vec(Context& c, const T* LU, int64_t ld, int cm, int64_t n, const int64_t* perm,
-                      T* X, int64_t ldx, int64_t nrhs, T* tmp, int trans, hipStream_t s)
+                      T* x, T* tmp, int trans, hipStream_t s)
 {
     T* d0 = dinv_pair<T>(c, n);
     T* d1 = d0 + trsv_aux_elems(n, int(sizeof(T)));
     const int t = trans ? 1 - cm : cm;                  // A^T = U^T L^T P^T: U^T is the lower one
     trsv_diag_inverse<T>(LU, ld, t, 1, trans ? 0 : 1, n, d0, s);
     trsv_diag_inverse<T>(LU, ld, t, 0, trans ? 1 : 0, n, d1, s);
-    for (int64_t j = 0; j < nrhs; ++j) {
-        T* x = X + j * ldx;
-        if (!trans) {
-            permute_convert<T, T>(x, tmp, perm, n, 0, s);
-            trsv_lookback<T>(LU, ld, t, 1, n, d0, tmp, tv_next(c, n), s);
-            trsv_lookback<T>(LU, ld, t, 0, n, d1, tmp, tv_next(c, n), s);
-        }
-        else {
-            trsv_lookback<T>(LU, ld, t, 1, n, d0, x, tv_next(c, n), s);
-            trsv_lookback<T>(LU, ld, t, 0, n, d1, x, tv_next(c, n), s);
-            permute_convert<T, T>(x, tmp, perm, n, 1, s);
-        }
-        copy_convert<T, T>(tmp, n, x, n, n, 1, s);
+    if (!trans) {
+        permute_convert<T, T>(x, tmp, perm, n, 0, s);
+        trsv_lookback<T>(LU, ld, t, 1, n, d0, tmp, tv_next(c, n), s);
+        trsv_lookback<T>(LU, ld, t, 0, n, d1, tmp, tv_next(c, n), s);
     }
+    else {
+        trsv_lookback<T>(LU, ld, t, 1, n, d0, x, tv_next(c, n), s);
+        trsv_lookback<T>(LU, ld, t, 0, n, d1, x, tv_next(c, n), s);
+        permute_convert<T, T>(x, tmp, perm, n, 1, s);
+    }
+    copy_convert<T, T>(tmp, n, x, n, n, 1, s);
 }
 
 template <class T>
@@ -1236,13 +1231,13 @@ template <class T>
 static void getrs_cm(Context& c, int trans, const T* A, int64_t lda, int64_t n, const int64_t* d_ipiv,
                      T* B, int64_t ldb, int64_t nrhs)
 {
-    if (nrhs <= VEC_RHS_MAX) {
+    if (nrhs == 1) {
         std::vector<int64_t> ip(n);
         SA_HIP(hipMemcpyAsync(ip.data(), d_ipiv, sizeof(int64_t) * n, hipMemcpyDeviceToHost, c.s0));
         SA_HIP(hipStreamSynchronize(c.s0));
         const int64_t* perm = upload_perm(c, ip.data(), n);
         c.rhs.ensure(sizeof(T) * size_t(n));
-        getrs_vec<T>(c, A, lda, 1, n, perm, B, ldb, nrhs, c.rhs.as<T>(), trans, c.s0);
+        getrs_vec<T>(c, A, lda, 1, n, perm, B, c.rhs.as<T>(), trans, c.s0);
         SA_HIP(hipStreamSynchronize(c.s0));
         check_kernel_error(c);
         return;
@@ -1268,7 +1263,7 @@ static int64_t potrf_cm(Context& c, int uplo, T* A, int64_t n, int64_t lda, cons
 template <class T>
 static void potrs_cm(Context& c, int uplo, T* A, int64_t lda, int64_t n, T* B, int64_t ldb, int64_t nrhs)
 {
-    if (nrhs <= VEC_RHS_MAX) {
+    if (nrhs == 1) {
         // Lower column-major L (A = L L^T): L y = b, L^T x = y.
         // Upper column-major U (A = U^T U): U^T y = b, U x = y.
         const int cmL = (uplo == SLATE_AMD_UPPER) ? 0 : 1;
@@ -1276,10 +1271,8 @@ static void potrs_cm(Context& c, int uplo, T* A, int64_t lda, int64_t n, T* B, i
         T* d1 = d0 + trsv_aux_elems(n, int(sizeof(T)));
         trsv_diag_inverse<T>(A, lda, cmL, 1, 0, n, d0, c.s0);
         trsv_diag_inverse<T>(A, lda, 1 - cmL, 0, 0, n, d1, c.s0);
-        for (int64_t j = 0; j < nrhs; ++j) {
-            trsv_lookback<T>(A, lda, cmL, 1, n, d0, B + j * ldb, tv_next(c, n), c.s0);
-            trsv_lookback<T>(A, lda, 1 - cmL, 0, n, d1, B + j * ldb, tv_next(c, n), c.s0);
-        }
+        trsv_lookback<T>(A, lda, cmL, 1, n, d0, B, tv_next(c, n), c.s0);
+        trsv_lookback<T>(A, lda, 1 - cmL, 0, n, d1, B, tv_next(c, n), c.s0);
         SA_HIP(hipStreamSynchronize(c.s0));
         check_kernel_error(c);
         return;

@@ -335,3 +335,47 @@ def test_batched_no_iterations(gpu):
         iters, info, _ = slate_amd.gesv_batched(ns, A, B, X, slate_amd.PREC_FP32,
                                                 opts=slate_amd.Options(max_iterations=most))
         assert (info == 0).all() and (iters == want).all()
+
+
+def _kernel_matrix(n, shift):
+    """A Gaussian kernel on n points plus a small diagonal: symmetric positive
+    definite, its diagonal blocks as ill conditioned as the whole."""
+    t = np.sort(np.random.default_rng(n).uniform(0, 1, n))
+    return np.exp(-((t[:, None] - t[None, :]) / 0.3) ** 2) + shift * np.eye(n)
+
+
+@pytest.mark.parametrize("n", [96, 256, 700])
+@pytest.mark.parametrize("nrhs", [2, 3, 4, 5])
+@pytest.mark.parametrize("kind", ["lu", "lu_t", "lu_float", "lower", "upper"])
+def test_few_right_hand_sides_backward_error(gpu, n, nrhs, kind):
+    """Solves of several right-hand sides substitute: the residual against the
+    computed factors stays below gamma_n for each triangle, entry by entry
+    (Higham, Accuracy and Stability, theorem 8.5), with no condition number.
+    |b - L U x| <= 2 n eps |L| |U| |x| holds both and the checking product."""
+    say("right-hand sides n=%d nrhs=%d %s" % (n, nrhs, kind))
+    dtype = torch.float32 if kind == "lu_float" else torch.float64
+    A = to_dev(_kernel_matrix(n, 1e-4 if kind == "lu_float" else 1e-10), dtype)
+    B = dev_rands(17, n, nrhs, dtype)
+    b = to_host(B)
+    if kind.startswith("lu"):
+        info, ipiv = slate_amd.getrf(A)
+        slate_amd.getrs(A, ipiv, B, trans=kind == "lu_t")
+        F = to_host(A)
+        L, U = np.tril(F, -1) + np.eye(n), np.triu(F)
+        perm = np.arange(n)
+        for i, p in enumerate(ipiv):
+            perm[i], perm[p - 1] = perm[p - 1], perm[i]
+    else:
+        uplo = slate_amd.LOWER if kind == "lower" else slate_amd.UPPER
+        info = slate_amd.potrf(A, uplo=uplo)
+        slate_amd.potrs(A, B, uplo=uplo)
+        F = to_host(A)
+        L = np.tril(F) if kind == "lower" else np.triu(F).T
+        U, perm = L.T, np.arange(n)
+    assert info == 0
+    x = to_host(B)
+    if kind == "lu_t":
+        r, bound = b - U.T @ (L.T @ x[perm]), np.abs(U.T) @ (np.abs(L.T) @ np.abs(x[perm]))
+    else:
+        r, bound = b[perm] - L @ (U @ x), np.abs(L) @ (np.abs(U) @ np.abs(x))
+    assert (np.abs(r) <= 2 * n * float(torch.finfo(dtype).eps) * bound).all()
