@@ -535,6 +535,21 @@ __device__ __forceinline__ double row_dot(const double* __restrict__ A, int n, i
     return ((ps[0] + ps[1]) + (ps[2] + ps[3])) + ((ps[4] + ps[5]) + (ps[6] + ps[7]));
 }
 
+// Norms keep NaN (fmax drops it): a factor or solution that overflowed has a
+// norm that is not finite, and such a norm never meets the tolerance.
+__device__ __forceinline__ double norm_max(double a, double b) { return (a > b || a != a) ? a : b; }
+__device__ __forceinline__ bool b_converged(double rnorm, double xnorm, double anorm, double tol)
+{
+    const double lim = xnorm * anorm * tol;
+    return isfinite(lim) && rnorm <= lim;
+}
+// ||b - A x|| / (||A|| ||x||), not finite where the solution is not.
+__device__ __forceinline__ double b_backward_error(double rnorm, double xnorm, double anorm)
+{
+    const double den = anorm * xnorm;
+    return den == 0 ? 0.0 : rnorm / den;
+}
+
 // r = b - A x (FP64, A column-major) and infinity norms: ||r|| in s_dred[0],
 // ||x|| in s_dred[1].  s_v: n doubles of LDS for x.
 template <int BT>
@@ -549,20 +564,20 @@ __device__ __forceinline__ void wg_residual(const double* __restrict__ A, int n,
     for (int i = tid; i < n; i += BT) {
         const double s = b[i] - row_dot<false>(A, n, i, s_v);
         r[i] = s;
-        rmax = fmax(rmax, fabs(s));
-        xmax = fmax(xmax, fabs(s_v[i]));
+        rmax = norm_max(rmax, fabs(s));
+        xmax = norm_max(xmax, fabs(s_v[i]));
     }
     #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
-        rmax = fmax(rmax, __shfl_xor(rmax, o, 64));
-        xmax = fmax(xmax, __shfl_xor(xmax, o, 64));
+        rmax = norm_max(rmax, __shfl_xor(rmax, o, 64));
+        xmax = norm_max(xmax, __shfl_xor(xmax, o, 64));
     }
     __syncthreads();
     if (lane == 0) { s_dred[2 + wave] = rmax; s_dred[2 + NW + wave] = xmax; }
     __syncthreads();
     if (tid == 0) {
         double a = 0, c = 0;
-        for (int w = 0; w < NW; ++w) { a = fmax(a, s_dred[2 + w]); c = fmax(c, s_dred[2 + NW + w]); }
+        for (int w = 0; w < NW; ++w) { a = norm_max(a, s_dred[2 + w]); c = norm_max(c, s_dred[2 + NW + w]); }
         s_dred[0] = a;
         s_dred[1] = c;
     }
@@ -578,20 +593,20 @@ __device__ __forceinline__ void wg_norms(const double* __restrict__ A, int n, co
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     double m = 0, vm = 0;
     for (int i = tid; i < n; i += BT) {
-        m = fmax(m, row_dot<true>(A, n, i, nullptr));
-        vm = fmax(vm, fabs(v[i]));
+        m = norm_max(m, row_dot<true>(A, n, i, nullptr));
+        vm = norm_max(vm, fabs(v[i]));
     }
     #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
-        m = fmax(m, __shfl_xor(m, o, 64));
-        vm = fmax(vm, __shfl_xor(vm, o, 64));
+        m = norm_max(m, __shfl_xor(m, o, 64));
+        vm = norm_max(vm, __shfl_xor(vm, o, 64));
     }
     __syncthreads();
     if (lane == 0) { s_dred[2 + wave] = m; s_dred[2 + NW + wave] = vm; }
     __syncthreads();
     if (tid == 0) {
         double a = 0, c = 0;
-        for (int w = 0; w < NW; ++w) { a = fmax(a, s_dred[2 + w]); c = fmax(c, s_dred[2 + NW + w]); }
+        for (int w = 0; w < NW; ++w) { a = norm_max(a, s_dred[2 + w]); c = norm_max(c, s_dred[2 + NW + w]); }
         s_dred[0] = a;
         s_dred[1] = c;
     }
@@ -763,10 +778,10 @@ __device__ __forceinline__ double wave_row_dot(const double* __restrict__ A, int
     return ((ps[0] + ps[1]) + (ps[2] + ps[3])) + ((ps[4] + ps[5]) + (ps[6] + ps[7]));
 }
 
-__device__ __forceinline__ double wave_fmax(double v)
+__device__ __forceinline__ double wave_norm_max(double v)
 {
     #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+    for (int o = 32; o > 0; o >>= 1) v = norm_max(v, __shfl_xor(v, o, 64));
     return v;
 }
 
@@ -808,11 +823,11 @@ __device__ __forceinline__ void wave_system(const BatchArgs& a, const double* gA
     auto residual = [&] {
         const double s = bl - wave_row_dot<false>(A, n, x);
         r = lane < n ? s : 0.0;
-        rnorm = wave_fmax(fmax(0.0, fabs(r)));
-        xnorm = wave_fmax(lane < n ? fmax(0.0, fabs(x)) : 0.0);
+        rnorm = wave_norm_max(fabs(r));
+        xnorm = wave_norm_max(lane < n ? fabs(x) : 0.0);
     };
-    const double anorm = wave_fmax(lane < n ? wave_row_dot<true>(A, n, 0.0) : 0.0);
-    const double bnorm = wave_fmax(fmax(0.0, fabs(bl)));
+    const double anorm = wave_norm_max(lane < n ? wave_row_dot<true>(A, n, 0.0) : 0.0);
+    const double bnorm = wave_norm_max(fabs(bl));
 
     int info = 0, iters = 0, ch = mode == 1 ? 2 : 1;
     bool need64 = mode == 1;
@@ -841,7 +856,7 @@ __device__ __forceinline__ void wave_system(const BatchArgs& a, const double* gA
             bool conv = false;
             for (int it = 0; it <= a.itermax; ++it) {
                 if (it > 0) residual();
-                conv = rnorm <= xnorm * anorm * tol;
+                conv = b_converged(rnorm, xnorm, anorm, tol);
                 if (conv) { iters = it; break; }
                 if (it == a.itermax) break;
                 x += wave_lu_solve<float>(s_f, n, lab, pl, diag, r);
@@ -864,8 +879,7 @@ __device__ __forceinline__ void wave_system(const BatchArgs& a, const double* gA
     if (lane == 0) {
         a.iters[sys] = iters;
         a.info[sys] = info;
-        const double den = anorm * xnorm;
-        a.berr[sys] = den > 0 ? rnorm / den : 0.0;
+        a.berr[sys] = b_backward_error(rnorm, xnorm, anorm);
         if (a.choice) a.choice[sys] = ch;
         if (a.ticks) a.ticks[sys] = wall_clock64() - t0;
     }
@@ -1028,7 +1042,7 @@ void batched_solve_kernel(BatchArgs a, char* gwork, const double* gA, const doub
                 continue;
             }
             // refinement: the residual of x is in r, its norms in s_dred
-            const bool conv = a.itermax >= 0 && s_dred[0] <= s_dred[1] * anorm * tol;
+            const bool conv = a.itermax >= 0 && b_converged(s_dred[0], s_dred[1], anorm, tol);
             __syncthreads();
             if (conv) { iters = it; break; }
             if (it >= a.itermax) {
@@ -1042,8 +1056,7 @@ void batched_solve_kernel(BatchArgs a, char* gwork, const double* gA, const doub
         if (tid == 0) {
             a.iters[sys] = iters;
             a.info[sys] = info;
-            const double den = anorm * s_dred[1];
-            a.berr[sys] = den > 0 ? s_dred[0] / den : 0.0;
+            a.berr[sys] = b_backward_error(s_dred[0], s_dred[1], anorm);
             if (a.choice) a.choice[sys] = ch;
             if (a.ticks) a.ticks[sys] = wall_clock64() - t0;
         }

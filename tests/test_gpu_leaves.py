@@ -379,3 +379,42 @@ def test_few_right_hand_sides_backward_error(gpu, n, nrhs, kind):
     else:
         r, bound = b[perm] - L @ (U @ x), np.abs(L) @ (np.abs(U) @ np.abs(x))
     assert (np.abs(r) <= 2 * n * float(torch.finfo(dtype).eps) * bound).all()
+
+
+@pytest.mark.parametrize("prec", [slate_amd.PREC_FP32, slate_amd.PREC_BF16])
+def test_batched_float_overflow_falls_back(gpu, prec):
+    """Entries above float's range make the float factor infinite or NaN: its
+    norms are not finite, so it does not count as converged, and the FP64
+    factor solves the system, on the one-wave and the workgroup path.  Scaling
+    a system by a number leaves its relative errors as they are, so the bound
+    is the one of the other batched tests."""
+    ns = [2, 40, 64, 65, 100, 300]
+    mats, rhs, A, B, X = _batch(ns, 8)
+    A *= 1e40
+    say("batched overflow, precision %d" % prec)
+    iters, info, berr = slate_amd.gesv_batched(ns, A, B, X, prec)
+    assert (info == 0).all() and (iters < 0).all()
+    assert (berr <= 32 * np.sqrt(np.asarray(ns)) * np.finfo(np.float64).eps).all()
+    x = X.cpu().numpy()
+    o = 0
+    for M, b, n in zip(mats, rhs, ns):
+        ref = np.linalg.solve(M, b)
+        np.testing.assert_allclose(1e40 * x[o:o + n], ref, rtol=0, atol=1e-11 * np.abs(ref).max())
+        o += n
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_batched_non_finite_is_reported(gpu, value):
+    """A non-finite entry in the matrix or the right-hand side never counts as
+    solved: no step count, and a backward error that is not finite."""
+    ns = [40, 40, 40, 100, 100, 100]
+    say("batched with %r" % value)
+    mats, rhs, A, B, X = _batch(ns, 9)
+    A[7] = value                       # systems 0 and 3: in the matrix
+    A[3 * 1600 + 7] = value
+    B[40 + 3] = value                  # systems 1 and 4: in the right-hand side
+    B[120 + 100 + 3] = value
+    iters, info, berr = slate_amd.gesv_batched(ns, A, B, X, slate_amd.PREC_FP32)
+    bad = np.array([True, True, False, True, True, False])
+    np.testing.assert_array_equal(iters < 0, bad)
+    np.testing.assert_array_equal(~np.isfinite(berr), bad)
