@@ -391,17 +391,6 @@ __device__ __forceinline__ void wg_getrf(T* __restrict__ W, int n, int ldw, int*
     }
 }
 
-// y / d from dinv = 1 / d: the product corrected by its residual, which rounds
-// as the division does; the division itself outside the range where dinv or
-// the residual would lose bits.
-__device__ __forceinline__ double b_quotient(double y, double d, double dinv)
-{
-    const double q = y * dinv;
-    double r = fma(fma(-q, d, y), dinv, q);
-    if (!(fabs(d) < 1e290 && fabs(dinv) < 1e290 && isfinite(r))) r = y / d;
-    return r;
-}
-
 // x := op(LU)^{-1} x for the factors in W (row-major), x of length n in
 // global memory (FP64).  Lower (unit) or upper, 64-row blocks: the diagonal
 // block is staged in LDS (s_blk, 64 x 65 T) and solved by wave 0 with
@@ -444,11 +433,25 @@ __device__ __forceinline__ void wg_trsv(const T* __restrict__ W, int n, int ldw,
                     }
                 }
                 else {
+                    // y stays the row's numerator; outside the quotients' range
+                    // the block is solved again with divisions
+                    const double y0 = y;
                     #pragma unroll 8
                     for (int j = bn - 1; j >= 0; --j) {
-                        const double yj = lane_val(b_quotient(y, d, dinv), j), u = double(row[j]);
-                        y = lane == j ? yj : lane < j ? y - u * yj : y;
+                        const double yj = lane_val(quot_by_inverse(y, d, dinv), j), u = double(row[j]);
+                        y = lane < j ? y - u * yj : y;
                     }
+                    double q = quot_by_inverse(y, d, dinv);
+                    if (__ballot(!(quot_range(d) && quot_holds(y, q)))) {
+                        y = y0;
+                        #pragma unroll 1
+                        for (int j = bn - 1; j >= 0; --j) {
+                            const double yj = lane_val(y / d, j), u = double(row[j]);
+                            y = lane < j ? y - u * yj : y;
+                        }
+                        q = y / d;
+                    }
+                    y = q;
                 }
             }
             if (lane < bn) x[b0 + lane] = y;
@@ -746,11 +749,22 @@ __device__ __forceinline__ double wave_lu_solve(const T* Fp, int n, int lab, int
         }
     }
     else {
+        // as in wg_trsv
+        const double y0 = y;
         #pragma unroll 8
         for (int k = n - 1; k >= 0; --k) {
-            const double xk = lane_val(b_quotient(y, d, dinv), __builtin_amdgcn_readlane(pl, k));
+            const double xk = lane_val(quot_by_inverse(y, d, dinv), __builtin_amdgcn_readlane(pl, k));
             y = lab < k ? y - double(F[64 * k + lane]) * xk : y;
             x = lane == k ? xk : x;
+        }
+        if (__ballot(!(quot_range(d) && quot_holds(y, quot_by_inverse(y, d, dinv))))) {
+            y = y0;
+            #pragma unroll 1
+            for (int k = n - 1; k >= 0; --k) {
+                const double xk = lane_val(y / d, __builtin_amdgcn_readlane(pl, k));
+                y = lab < k ? y - double(F[64 * k + lane]) * xk : y;
+                x = lane == k ? xk : x;
+            }
         }
     }
     return x;

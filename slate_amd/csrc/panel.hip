@@ -138,9 +138,6 @@ struct alignas(4 * sizeof(T)) LeafHead { T val, fac, nxt; uint32_t idx; };
 template <class T>
 struct LeafDec { LeafHead<T> h; T u2; };
 
-__device__ __forceinline__ double fma_of(double a, double b, double c) { return __builtin_fma(a, b, c); }
-__device__ __forceinline__ float fma_of(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-
 // Of E candidates in LDS, the largest magnitude, then the smallest row.
 template <class T>
 __device__ __forceinline__ int leaf_best(const LeafHead<T>* h, int E)

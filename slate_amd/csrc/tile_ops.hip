@@ -129,9 +129,9 @@ template void trsm_leaf<float>(const float*, int64_t, int, int, int, int64_t, fl
 // form needs 2 m/32 - 1 launches.
 // Non-unit diagonals: 32 dependent divisions per block are as long as the
 // rest of the substitution, so each row's reciprocal is formed once, off the
-// chain, and the quotient is corrected by its residual, which rounds as the
-// division does; blocks with a diagonal entry outside the range where that
-// holds divide.
+// chain, and corrected quotients take their place (quot_by_inverse).  A wave
+// that meets a diagonal entry, a numerator or a quotient outside the range
+// where these round as divisions solves its block again with divisions.
 template <class T> __device__ __forceinline__ T bcast_half(T v, int k, bool upper);
 template <> __device__ __forceinline__ float bcast_half<float>(float v, int k, bool upper)
 {
@@ -296,30 +296,29 @@ void trsm_fused_kernel(TrsmProb<T> P)
             }
         }
         else {
-            constexpr T big = sizeof(T) == 8 ? T(1e290) : T(1e30);
-            const T inv = T(1) / diag;
-            if (__ballot(!(fabs(diag) < big && fabs(inv) < big)) == 0) {
+            const T inv = T(1) / diag, y0 = y;
+            // y stays the row's numerator; after step r so does its quotient x
+            T x = T(0);
+            #pragma unroll
+            for (int k = 0; k < 32; ++k) {
+                x = quot_by_inverse(y, diag, inv);
+                if (k < 31) {
+                    const T xk = bcast_half<T>(x, k, upper);
+                    if (r > k) y -= lr[k] * xk;
+                }
+            }
+            if (__ballot(!(quot_range(diag) && quot_holds(y, x)))) {
+                x = y0;
                 #pragma unroll
                 for (int k = 0; k < 32; ++k) {
-                    const T q0 = y * inv;
-                    const T q1 = fma(fma(-q0, diag, y), inv, q0);
-                    if (r == k) y = isfinite(q1) ? q1 : q0;
+                    if (r == k) x = x / diag;
                     if (k < 31) {
-                        const T xk = bcast_half<T>(y, k, upper);
-                        if (r > k) y -= lr[k] * xk;
+                        const T xk = bcast_half<T>(x, k, upper);
+                        if (r > k) x -= lr[k] * xk;
                     }
                 }
             }
-            else {
-                #pragma unroll
-                for (int k = 0; k < 32; ++k) {
-                    if (r == k) y = y / diag;
-                    if (k < 31) {
-                        const T xk = bcast_half<T>(y, k, upper);
-                        if (r > k) y -= lr[k] * xk;
-                    }
-                }
-            }
+            y = x;
         }
         if (i < m) Xc[i] = y;
     }

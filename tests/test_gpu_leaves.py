@@ -418,3 +418,47 @@ def test_batched_non_finite_is_reported(gpu, value):
     bad = np.array([True, True, False, True, True, False])
     np.testing.assert_array_equal(iters < 0, bad)
     np.testing.assert_array_equal(~np.isfinite(berr), bad)
+
+
+# numerators and quotients near both ends of the range, subnormal ones among
+# them, where a product with the reciprocal and one correction would lose bits
+_EXTREME = {np.float64: [1e-290, 1e-300, 5e-308, 1e-310, 3e-320, 1e306, 1.0, 0.0],
+            np.float32: [1e-30, 1e-36, 3e-38, 1e-40, 3e-44, 1e37, 1.0, 0.0]}
+
+
+def _extreme_quotients(n, T, seed):
+    rng = np.random.default_rng(seed)
+    d = rng.uniform(1, 16, n).astype(T)
+    b = np.stack([(rng.uniform(1, 2, n) * s).astype(T) for s in _EXTREME[T]], axis=1)
+    return d, b, b / d[:, None]
+
+
+@pytest.mark.parametrize("T", [np.float64, np.float32])
+@pytest.mark.parametrize("trans", [False, True])
+def test_getrs_extreme_numerators(gpu, T, trans):
+    """A diagonal factor: every entry is one division, correctly rounded (the
+    other terms of the substitution are exact zeros)."""
+    say("getrs extreme numerators %s trans=%s" % (T.__name__, trans))
+    n = 70
+    dtype = torch.float64 if T is np.float64 else torch.float32
+    d, b, ref = _extreme_quotients(n, T, 3)
+    B = slate_amd.colmajor(torch.from_numpy(np.asfortranarray(b)).to(dtype).cuda())
+    slate_amd.getrs(slate_amd.colmajor(torch.from_numpy(np.diag(d)).cuda()), np.arange(1, n + 1), B, trans=trans)
+    np.testing.assert_array_equal(B.cpu().numpy(), ref)
+
+
+def test_batched_extreme_numerators(gpu):
+    """The same for the FP64 solves of the batch, one wave and a workgroup."""
+    say("batched extreme numerators")
+    ns, mats, rhs, refs = [], [], [], []
+    for n in (33, 64, 100):
+        d, b, ref = _extreme_quotients(n, np.float64, n)
+        for j in range(b.shape[1]):
+            ns.append(n)
+            mats.append(np.diag(d).ravel())
+            rhs.append(b[:, j])
+            refs.append(ref[:, j])
+    X = torch.zeros(sum(ns), dtype=torch.float64, device="cuda")
+    slate_amd.gesv_batched(ns, torch.from_numpy(np.concatenate(mats)).cuda(), torch.from_numpy(np.concatenate(rhs)).cuda(),
+                           X, slate_amd.PREC_FP64)
+    np.testing.assert_array_equal(X.cpu().numpy(), np.concatenate(refs))
