@@ -122,8 +122,6 @@ def test_panel_leaf_non_finite(gpu, value, n):
     np.testing.assert_array_equal(np.sort(a[20:], axis=0), np.sort(b[20:], axis=0))
 
 
-# 32 x 64 tiles (few tiles), 64 x 64 and 128 x 128 tiles, each with whole
-# tiles, ragged edges, a k tail, and operands one element off 16-byte alignment
 @pytest.mark.parametrize("n,dtype", [(520, torch.float64), (8321, torch.float64), (28801, torch.float64),
                                      (8321, torch.float32), (28801, torch.float32)])
 def test_panel_leaf_exchange_shapes(gpu, n, dtype):
@@ -194,6 +192,8 @@ def test_panel_leaf_zero_column(gpu):
     assert info == 41 and ipiv[40] == 41
 
 
+# 32 x 64 tiles (few tiles), 64 x 64 and 128 x 128 tiles, each with whole
+# tiles, ragged edges, a k tail, and operands one element off 16-byte alignment
 @pytest.mark.parametrize("m,n,k", [(70, 130, 200), (64, 128, 128), (1100, 1000, 70), (1088, 1024, 64),
                                    (2100, 2050, 33), (2048, 2176, 48)])
 @pytest.mark.parametrize("off", [0, 1])
@@ -462,3 +462,71 @@ def test_batched_extreme_numerators(gpu):
     slate_amd.gesv_batched(ns, torch.from_numpy(np.concatenate(mats)).cuda(), torch.from_numpy(np.concatenate(rhs)).cuda(),
                            X, slate_amd.PREC_FP64)
     np.testing.assert_array_equal(X.cpu().numpy(), np.concatenate(refs))
+
+
+def _lu_error(A, F, ipiv, rows=None):
+    """(|L| below the diagonal by column, whether |P A - L U| <= 2 n eps |L| |U|
+    on the rows): n eps for the factorization, as much for the product here.
+    A: the matrix, F: its factors, on the device."""
+    n = A.shape[0]
+    perm = np.arange(n)
+    for i, p in enumerate(ipiv):
+        perm[i], perm[p - 1] = perm[p - 1], perm[i]
+    rows = torch.arange(n, device="cuda") if rows is None else torch.from_numpy(rows).cuda()
+    L = torch.where(rows[:, None] > torch.arange(n, device="cuda")[None, :], F[rows], 0)
+    most = L.abs().amax(0)
+    L[torch.arange(len(rows), device="cuda"), rows] = 1.0
+    U = F.triu()
+    r = A[torch.from_numpy(perm).cuda()[rows]] - L @ U
+    return most, bool((r.abs() <= 2 * n * torch.finfo(F.dtype).eps * (L.abs() @ U.abs())).all())
+
+
+@pytest.mark.parametrize("n,ld", [(700, 700), (700, 701), (1500, 1504)])
+@pytest.mark.parametrize("ib", [5, 16, 20, 32])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_panel_leaf_exchange_widths(gpu, n, ld, ib, dtype):
+    """Leaves across workgroups in both register forms (16 and 32 columns) and
+    narrower than them, rows aligned and not: pivoted strictly, the oracle's
+    pivots in FP64, P A = L U."""
+    say("panel leaf exchange n=%d ld=%d ib=%d %s" % (n, ld, ib, dtype))
+    A = dev_rands(12, n, n, dtype)
+    F = slate_amd.empty_colmajor(n, n, dtype, ld=ld)
+    F.copy_(A)
+    info, ipiv = slate_amd.getrf(F, slate_amd.Options(block_size=128, inner_blocking=ib))
+    assert info == 0
+    most, close = _lu_error(A, F, ipiv)
+    assert float(most.max()) <= 1.0 and close
+    if dtype == torch.float64:
+        np.testing.assert_array_equal(ipiv, oracle.getrf(oracle.rands(12, n, n), nb=128, ib=16)[1])
+
+
+@pytest.mark.parametrize("n,ib", [(33001, 0), (57400, 32)])
+def test_panel_leaf_tall(gpu, n, ib):
+    """FP64 panels above 32768 rows, where leaves of 16 columns keep two rows
+    per thread, and above 57344 rows with 32 columns and two rows per thread:
+    pivoted strictly, P A = L U on rows from the top, the middle and the end."""
+    say("panel leaf n=%d ib=%d" % (n, ib))
+    g = torch.Generator("cuda").manual_seed(n)
+    A = torch.empty(n, n, dtype=torch.float64, device="cuda").uniform_(-1, 1, generator=g).t()
+    F = A.t().clone().t()
+    info, ipiv = slate_amd.getrf(F, slate_amd.Options(inner_blocking=ib))
+    assert info == 0
+    most, close = _lu_error(A, F, ipiv, np.r_[0:100, n // 2:n // 2 + 50, n - 100:n])
+    assert float(most.max()) <= 1.0 and close
+
+
+@pytest.mark.parametrize("n", [300, 700, 1500])
+def test_panel_leaf_threshold_factors(gpu, n):
+    """With a threshold of 0.5 a column whose diagonal was kept has |L| <= 2 up
+    to the rounding of the scaling, one that was interchanged |L| <= 1 (both
+    kinds occur), and P A = L U with the pivots taken, whatever they are."""
+    say("panel leaf threshold factors n=%d" % n)
+    A = dev_rands(77, n, n)
+    F = A.t().clone().t()
+    info, ipiv = slate_amd.getrf(F, slate_amd.Options(pivot_threshold=0.5, block_size=128))
+    assert info == 0
+    most, close = _lu_error(A, F, ipiv)
+    kept = torch.from_numpy(ipiv == np.arange(1, n + 1)).cuda()
+    assert 0 < int(kept.sum()) < n
+    assert float(most[kept].max()) <= 2 * (1 + 4 * np.finfo(np.float64).eps)
+    assert float(most[~kept].max()) <= 1.0 and close
