@@ -229,14 +229,6 @@ __device__ __forceinline__ int wave_argmax_lane(T v, uint32_t idx, uint32_t key,
     }
     return __builtin_ctzll(eq);
 }
-template <class T>
-__device__ __forceinline__ void wave_argmax(T& v, uint32_t& idx)
-{
-    const uint32_t key = argmax_key(v);
-    const int lane = wave_argmax_lane(v, idx, key, wave_max_u32(key));
-    v = lane_val(v, lane);
-    idx = uint32_t(__builtin_amdgcn_readlane(int(idx), lane));
-}
 
 // y / d from inv = 1 / d, which is formed off the chain of a substitution: the
 // product corrected by its residual.  With d, y and the quotient in quot_range

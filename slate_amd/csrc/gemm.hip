@@ -611,8 +611,10 @@ void gemm(const GemmArgs& a, int alay, int blay, hipStream_t s, int role)
     }
     else if (alay == A_KC && blay == B_NC) launch<T, A_KC, B_NC>(a, s);
     else if (alay == A_MC && blay == B_NC) launch<T, A_MC, B_NC>(a, s);
-    else if (alay == A_KC && blay == B_KC) launch<T, A_KC, B_KC>(a, s);
-    else launch<T, A_MC, B_KC>(a, s);
+    else {
+        SA_REQUIRE(alay == A_KC && blay == B_KC, -2, "gemm: no product of two transposed operands");
+        launch<T, A_KC, B_KC>(a, s);
+    }
 }
 
 template void gemm<double>(const GemmArgs&, int, int, hipStream_t, int);

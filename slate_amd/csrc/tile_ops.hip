@@ -379,19 +379,6 @@ template void trsm_fused<float>(const float*, int64_t, int, int, int, int64_t, f
 // 64 x 64 FP64 alone 33 us, FP32 beside the trailing updates of an
 // n = 16384 posv_mixed 54 us; four waves sharing the update from LDS, with
 // three barriers per column, took 86 and 89 us.
-template <class T> __device__ __forceinline__ T wave_bcast(T v, int lane);
-template <> __device__ __forceinline__ float wave_bcast<float>(float v, int lane)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
-}
-template <> __device__ __forceinline__ double wave_bcast<double>(double v, int lane)
-{
-    const uint64_t u = __builtin_bit_cast(uint64_t, v);
-    const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(u)), lane));
-    const uint32_t hi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(u >> 32)), lane));
-    return __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
-}
-
 // Steps [k, kend) with C live register rows (k + C >= 64 on entry); returns
 // false at a non-positive pivot, with k the failing step.
 template <class T, int C>
@@ -400,7 +387,7 @@ __device__ __forceinline__ bool potrf_leaf_steps(T* __restrict__ A, int64_t ld, 
 {
     #pragma unroll 1
     for (; k < kend; ++k) {
-        const T d = wave_bcast<T>(v[0], k);
+        const T d = lane_val(v[0], k);
         if (!(d > T(0))) return false;
         const T dk = sqrt(d);
         T u = lane == k ? dk : v[0] / dk;
