@@ -124,9 +124,15 @@ __device__ __forceinline__ void wg_load_rowmajor(const double* __restrict__ A, i
 // tile took 32 loads and 32 stores, and two tiles in flight already exceeded
 // the 63 a wave can have outstanding.  A wave takes a strip of tiles, keeps
 // the strip's U (NB x 16 VE) in registers and has the next tile's loads
-// (clamped, unguarded) in flight during the products.  Lane l's k-steps are
-// consecutive, too (k = (NB/4) (l/16) + s): L fragments are 16-byte reads.
+// (clamped, unguarded) in flight during the products.  Step s takes the
+// products k = 4 s .. 4 s + 3, lane l the one of k = 4 s + l/16, so each sum
+// runs in the order of k (rows of U grow with k: any other order has larger
+// partial sums, 1.15 times the error of the FP32 factor of a uniform matrix);
+// a row of L holds the columns 4 s + g at (NB/4) g + s (lds_column), so that a
+// lane's are consecutive and L fragments are 16-byte reads.
 // Row of accumulator register r: 4 r + l/16 (FP64), 4 (l/16) + r (FP32).
+template <int NB> constexpr int lds_column(int p) { return 4 * (p % (NB / 4)) + p / (NB / 4); }
+
 template <class T, int NB, int LD, int BT, bool BFU>
 __device__ __forceinline__ void wg_update(T* __restrict__ C, const T* __restrict__ U, int ldw, const T* __restrict__ L,
                                           int nr)
@@ -145,9 +151,9 @@ __device__ __forceinline__ void wg_update(T* __restrict__ C, const T* __restrict
     for (int it = wave; it < tc * parts; it += NW) {
         const int t0 = (it / tc) * per, t1 = min(tr, t0 + per);
         const int jv = (it % tc) * 16 * VE + VE * fr, jc = min(jv, lastv);
-        vec_t bv[KS];                                   // U rows k = KS fg + s, element b for block b
+        vec_t bv[KS];                                   // U rows k = 4 s + fg, element b for block b
         #pragma unroll
-        for (int s = 0; s < KS; ++s) bv[s] = *reinterpret_cast<const vec_t*>(U + (KS * fg + s) * ldw + jc);
+        for (int s = 0; s < KS; ++s) bv[s] = *reinterpret_cast<const vec_t*>(U + (4 * s + fg) * ldw + jc);
         vec_t cv[2][2][4];
         auto fetch = [&](int set, int t) {
             #pragma unroll
@@ -265,7 +271,8 @@ __device__ __forceinline__ void wg_getrf(T* __restrict__ W, int n, int ldw, int*
                 }
             }
             leaf_wg_factor<T, NB, RPT, BT>(s_leaf, v, lab, kb, mr, W, ldw, k0, k0, s_info, T(1));
-            // rows to their places, in memory and in LDS; v[q][c] holds column (kb + c) mod NB
+            // rows to their places, in memory and in LDS (L11 in the order of its
+            // columns, L21 as wg_update reads it); v[q][c] holds column (kb + c) mod NB
             #pragma unroll
             for (int q = 0; q < RPT; ++q) {
                 const int i = lab[q];
@@ -279,7 +286,16 @@ __device__ __forceinline__ void wg_getrf(T* __restrict__ W, int n, int ldw, int*
                         #pragma unroll
                         for (int e = 0; e < VE; ++e) x[e] = v[q][c + e];
                         *reinterpret_cast<vec_t*>(rowp + c) = x;
-                        *reinterpret_cast<vec_t*>(sp + c) = x;
+                        if (i < NB) *reinterpret_cast<vec_t*>(sp + c) = x;
+                    }
+                    if (i >= NB) {
+                        #pragma unroll
+                        for (int c = 0; c < NB; c += VE) {
+                            vec_t x;
+                            #pragma unroll
+                            for (int e = 0; e < VE; ++e) x[e] = v[q][lds_column<NB>(c + e)];
+                            *reinterpret_cast<vec_t*>(sp + c) = x;
+                        }
                     }
                 }
                 else {

@@ -3,6 +3,8 @@ the Cholesky leaf (64 x 64, four register stages of 16 rows) and the inverted
 diagonal blocks of the look-back solves (64 rows FP64, 128 rows FP32, four
 stages), and the LU panel leaf (one workgroup up to 512 rows, an exchange of up
 to 128 above)."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -530,3 +532,30 @@ def test_panel_leaf_threshold_factors(gpu, n):
     assert 0 < int(kept.sum()) < n
     assert float(most[kept].max()) <= 2 * (1 + 4 * np.finfo(np.float64).eps)
     assert float(most[~kept].max()) <= 1.0 and close
+
+
+@pytest.mark.parametrize("cfg", [(16, 256), (32, 256), (16, 512)])
+@pytest.mark.parametrize("prec", [slate_amd.PREC_FP32, slate_amd.PREC_FP64])
+def test_batched_update_order(gpu, cfg, prec):
+    """The trailing update sums its products in the order of k.  Here the first
+    two cancel, 2^23 - 2^23 (2^52 in FP64), before products of 1/4 arrive, so
+    the factor is exact in that order and in others loses the small ones; an
+    exact factor solves the system without a refinement step, bit for bit."""
+    say("batched update order %s precision %d" % (cfg, prec))
+    n, big = 80, 2.0 ** (23 if prec == slate_amd.PREC_FP32 else 52)
+    M = np.eye(n)
+    M[0, 32:], M[1, 32:], M[4, 32:], M[8, 32:] = big, -big, 0.25, 0.25
+    M[32:, [0, 1, 4, 8]] = 1.0
+    M[32:, 32:] = 0.5 + 4.0 * np.eye(n - 32)
+    x = np.r_[np.arange(1.0, 33.0), np.tile([1.0, -1.0], (n - 32) // 2)]
+    A = torch.from_numpy(M.T.ravel().copy()).cuda()
+    B = torch.tensor([math.fsum(row * x) for row in M], dtype=torch.float64, device="cuda")
+    X = torch.zeros_like(B)
+    saved = slate_amd.tune_get_batched()[:3]
+    try:
+        slate_amd.tune_set_batched(*cfg, 1)
+        iters, info, _ = slate_amd.gesv_batched([n], A, B, X, prec)
+    finally:
+        slate_amd.tune_set_batched(*saved)
+    assert info[0] == 0 and iters[0] == 0
+    np.testing.assert_array_equal(X.cpu().numpy(), x)
