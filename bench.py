@@ -410,7 +410,7 @@ def main():
     fp8 = args.factor_precision.startswith("fp8")
     f64 = args.factor_precision == "fp64"
     if f64:
-        names[S.PROF_OTHER] = "gemm_vec_kernel<double, 128, 128, 1, 1> trailing update (v_mfma_f64_16x16x4f64, FP64 LU)"
+        names[S.PROF_OTHER] = "gemm_vec_kernel<double, 0, 128, 128, 1, 1> trailing update (v_mfma_f64_16x16x4f64, FP64 LU)"
     if fp8:
         names[S.PROF_OTHER] = ("gemm_f8_kernel<%d,1> trailing update (e4m3 planes with a power-of-two scale per "
                                "tile, v_mfma_scale_f32_16x16x128_f8f6f4, %d products per update)"

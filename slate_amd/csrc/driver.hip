@@ -694,10 +694,14 @@ static void getrf_rm(Context& c, T* A, int64_t n, int64_t ld, const Opts& o, int
             panel_nopiv<T>(c, A, ld, n, p0, pw, ipiv, info, leaf_w, plan1, npu, npt, s1);
         }
         else {
-            // FP64 panels taller than 32768 rows keep 16-column leaves: there
-            // the 32-column form leaves no second workgroup on a CU
-            // (measured 3564 -> 3980 ms at n = 65536), while below it the
-            // wider leaves save launches (643 -> 625 ms at n = 32768).
+            // FP64 panels taller than 32768 rows take 16-column leaves.  Above
+            // 57344 rows 32 columns need two rows of 256 bytes per thread,
+            // which fit no place of a GEMM workgroup; down to 32768 rows the
+            // two widths are within 1.5%, below it the wider leaves win (half
+            // the launches).  getrf with 16 and with 32 columns throughout,
+            // ms: n = 16384 114 and 107, 32768 503 and 482; with 16 and with
+            // 32 above 32768 rows only: 40000 834 and 838, 49152 1404 and
+            // 1416, 57344 2156 and 2179, 65536 3131 and 3545.
             const bool narrow = n - p0 > 32768;
             const int64_t lw = (sizeof(T) == 8 && !c.calu && narrow && leaf_w > 16 && o.ib <= 0) ? 16 : leaf_w;
             panel_rec<T>(c, A, ld, n, p0, pw, ipiv, info, o.threshold, lw, plan1, s1, p0, pw);
@@ -890,7 +894,7 @@ static void potrf_rm(Context& c, T* A, int64_t n, int64_t ld, const Opts& o, int
                 return;
             }
         }
-        // U^T copied K-contiguous so the update runs on the 16-byte-staged kernel
+        // U^T copied K-contiguous; the update's kernel would stage it as it lies, too
         wk.ensure(sizeof(T) * size_t(r) * size_t(kb));
         T* ut = wk.as<T>();
         transpose_convert<T, T>(U, ld, ut, kb, r, kb, st);               // ut[i*kb + k] = U[k][i]
