@@ -96,7 +96,7 @@ struct Context {
     unsigned char* scratch = nullptr;   // this device's no-allocation scratch (noalloc.hip)
     Buf swaptmp;                 // two-pass row interchange workspace (trailing-update stream)
     Buf swaptmp1;                // the same for the lookahead block (tall blocks only)
-    Buf ttri;                    // diagonal block of a solve with few right-hand sides, row-major
+    Buf ttri;                    // diagonal block of a solve with several right-hand sides, row-major
     Buf cut0, cut1;              // Cholesky: K-contiguous U12^T for the trailing (s0) and block-row (s1) updates
     uint32_t tv_tag = 0;         // next free tag of tvw
     bool calu = false;           // leaves use tournament pivoting (MethodLU::CALU)
@@ -262,8 +262,8 @@ static void check_kernel_error(Context& c)
 // Recursive triangular solve with an nb x nb triangle and an nb x N row-major
 // right-hand side; off-diagonal blocks go through the MFMA GEMM.
 // tri(i,k) = M[i*ld + k] (cm = 0) or M[i + k*ld] (cm = 1).
-// tri (TRSM_TRI^2 elements, or null) is for solves with few right-hand sides
-// against a large triangle: diagonal blocks of at most TRSM_TRI rows, which a
+// tri (TRSM_TRI^2 elements, or null) is for the solves of a user's right-hand
+// sides (getrs, potrs): diagonal blocks of at most TRSM_TRI rows, which a
 // column-major view copies there row-major.  With 64 right-hand sides a
 // 512-row block in one launch has 8 workgroups and takes 245 us read by
 // columns; two of 256 rows and the product between them take about 80.
